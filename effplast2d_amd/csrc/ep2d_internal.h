@@ -7,6 +7,7 @@
 #include <cstdint>
 #include <stdexcept>
 #include <string>
+#include <vector>
 
 namespace ep2d {
 
@@ -179,6 +180,63 @@ constexpr int wide_cols(int ns) { return 128 - 4 * ns; }
 int wide_segments(int ns, int nX, int nY, int rows, int rve, int4* out);
 void launch_wide(int ns, const RveDev* rves, const int4* segs, int nsegs, int parity, int vpar,
                  hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
+// ---- resident runs (ep2d_resident.hip) ---------------------------------------
+// Shape of a tile's workgroup: waves of `rows` rows each (64 columns), and the
+// iterations between two exchanges with the neighbouring tiles.
+// cost: half CUs a tile is given (2: one tile to a CU); from: smallest grid.
+struct ResShape {
+  int rows = 0, every = 1, waves = 8, cost = 2, from = 0;
+};
+// One tile: own columns [i0, i1) and rows [j0, j1) of RVE rve; lane 0 is
+// column s, the first wave's first row is jr.  xl, xr, xu, xd: places of its
+// four edges in the exchange buffer, in pairs of words (16 bytes; -1: the edge
+// of the grid).
+struct ResTile {
+  int rve, s, i0, i1, jr, j0, j1;
+  int xl, xr, xu, xd;
+  int pad;
+};
+// Arrivals and departures of a launch's workgroups and how it went; zero
+// between launches.
+struct ResCtl {
+  unsigned arrive, state, depart, pad;
+};
+// how a launch went: run, or ended with the fields untouched because other
+// launches hold the GPU's room or its tiles did not all start in time; lost:
+// a wait inside the run ended at its bound (the fields are not valid)
+constexpr unsigned kResGo = 1, kResNoRoom = 2, kResLate = 3, kResLost = 4;
+constexpr long kResMinIters = 16;  // shorter runs take the other kernels
+constexpr int kResMinSide = 16;
+struct ResLaunch {
+  int mode;                 // scheme (1 or 2)
+  ResShape shape;
+  const RveDev* rves;
+  const ResTile* list;
+  int tiles;
+  int parity, vpar;         // U is read from U[parity ^ cur], V from Vx/Vy (0) or Vx2/Vy2
+  int iters;
+  char* xch;                // exchange buffer: two halves of xpar bytes
+  unsigned xpar;
+  unsigned tag0;            // tags tag0 + 1 .. tag0 + iters, none used before
+  ResCtl* ctl;
+  unsigned cost, room;      // half CUs of a tile, and of the device
+  unsigned* told;           // pinned host word that receives how the launch went
+};
+// The shapes of a scheme, from the smallest tiles to the largest: a grid takes
+// the first whose tiles find room together.
+std::vector<ResShape> resident_shapes(int mode);
+// Tiles of an n x n RVE (0: the shape does not fit it), its edges from pair x0
+// of the exchange buffer on; fills out when it is not null and gives the
+// pairs of one half the RVE's edges take.
+int resident_tiles(const ResShape& sh, int mode, int n, int rve, size_t x0, ResTile* out,
+                   size_t* pairs);
+int resident_room(int device);                        // half CUs
+int resident_cost(const ResShape& sh, int mode);      // half CUs of a tile (0: does not fit)
+// `iters` iterations of every RVE of the list: U[cur] receives U before the
+// last iteration, U[cur ^ 1] U after it, V is updated in place.
+void launch_resident(const ResLaunch& a, hipStream_t s, hipEvent_t e0 = nullptr,
+                     hipEvent_t e1 = nullptr);
+
 // batched fused iteration over many RVEs: tiles[k] = (rve, i0, j0, parity
 // offset); RVE k reads U[parity ^ offset].  All RVEs share mode and tile height.
 void launch_fused_batch(const RveDev* rves, const int4* tiles, int ntiles, int mode, int ty,

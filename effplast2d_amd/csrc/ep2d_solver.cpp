@@ -274,19 +274,27 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
   for (double* p : {f_.P, f_.tauXX, f_.tauYY, f_.tauXYav, f_.J2}) launch_fill(p, nC, 0.0, stream_);
   for (double* p : {f_.tauXY, f_.J2XY}) launch_fill(p, nV, 0.0, stream_);
   buildGatherTable();
+  // (not on a caller's stream: launches captured there are replayed on the
+  // buffers they were captured with, which a run of an even number of the tile
+  // kernel's iterations leaves current and the other kernels may not)
+  const bool autoShape = fused && ownStream_ && opt_.tileRows == 0 && opt_.marchRows == 0 &&
+                         opt_.itersPerLaunch == 0 && opt_.laneColumns == 0 &&
+                         opt_.stageWaves == 0;
   if (fused && opt_.tileRows == 0 && opt_.marchRows == 0 && opt_.itersPerLaunch == 0) {
-    // automatic shape for one RVE, from one-RVE measurements: both schemes
-    // from 1024^2 on four-stage chains with two waves per stage (four
-    // iterations per launch, in the launch order of chain_work_order): at
-    // 1024^2 the shortest segments whose workgroups the device holds in one
-    // round (14 rows for split, 21 for FP64 on 256 CUs: 7.4 and 15.6 us per
-    // iteration; 16 split rows take 8.6, 20 FP64 rows 17.3 and the FP64
-    // tile kernel 16.7), 48 rows at 2048^2 and 96 beyond (split 16.4 and
-    // 57.6 us, FP64 43.0 and 124.3 against 47.6 and 154.7 on wave pairs);
-    // the tile kernel below 1024^2.
+    // automatic shape for one RVE, from one-RVE measurements: four-stage
+    // chains with two waves per stage (four iterations per launch, in the
+    // launch order of chain_work_order).  Up to 1024^2 the shortest segments
+    // whose workgroups the device holds in one round (14 rows for split, 21
+    // for FP64 on 256 CUs at 1024^2: 7.1 and 14.7 us per iteration; 16 split
+    // rows take 8.6, 20 FP64 rows 17.3 and the FP64 tile kernel 16.7; at
+    // 1000^2 7.1 and 14.7 against 13.2 and 18.4 on the tile kernel, at 256^2
+    // 3.6 and 6.0 against 6.0 and 6.8), 48 rows at 2048^2 and 96 beyond
+    // (split 16.4 and 57.6 us, FP64 43.0 and 124.3 against 47.6 and 154.7 on
+    // wave pairs).  Runs of kResMinIters iterations and more of a grid that
+    // fits on the chip take the resident kernel (planResident) instead.
     const int n = std::max(nX, nY);
-    const bool chains = (mode_ == EP2D_MODE_SPLIT || mode_ == EP2D_MODE_FP64) && n >= 1024 &&
-                        multi_iter_fits(nX, nY) &&
+    const bool chains = (mode_ == EP2D_MODE_SPLIT || mode_ == EP2D_MODE_FP64) &&
+                        (n >= 1024 || (autoShape && !pool_)) && multi_iter_fits(nX, nY) &&
                         !(mode_ == EP2D_MODE_FP64 && opt_.laneColumns == 2);
     if (chains) {
       int rows = n <= 2048 ? 48 : 96;
@@ -294,11 +302,13 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
         const int cols = chain_cols(4, 2);
         const int strips = (nX + cols - 1) / cols;
         const int bands = std::max(1, chain_resident(4, 2, mode_ == EP2D_MODE_SPLIT) / strips);
-        rows = std::max(8, (nY + bands - 1) / bands);
+        rows = std::max(2, (nY + bands - 1) / bands);
       }
       opt_.marchRows = rows;
       opt_.itersPerLaunch = 4;
       if (opt_.laneColumns != 2 && opt_.stageWaves == 0) opt_.stageWaves = 2;
+      // one iteration on its own: the tile kernel below 1024^2
+      tileSingles_ = n < 1024;
     }
   }
   if (fused) {
@@ -326,15 +336,10 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
       // on the device (the kernel reads the current buffer as parity ^ cur)
       marchRows_ = opt_.marchRows;
       nSegs_ = march_segments(nX, nY, marchRows_, 0, nullptr);
-      std::vector<int4> segs((size_t)nSegs_);
+      std::vector<int4> segs((size_t)nSegs_), s2, c3, c2;
       march_segments(nX, nY, marchRows_, 0, segs.data());
-      dRve_ = (RveDev*)alloc(sizeof(RveDev));
-      dSegs_ = (int4*)alloc(segs.size() * sizeof(int4));
-      RveDev rd = r_;
-      rd.cur = 0;
-      EP2D_HIP(hipMemcpyAsync(dRve_, &rd, sizeof(RveDev), hipMemcpyHostToDevice, stream_));
-      EP2D_HIP(hipMemcpyAsync(dSegs_, segs.data(), segs.size() * sizeof(int4),
-                              hipMemcpyHostToDevice, stream_));
+      const int2 dims = make_int2(nX, nY);
+      const bool f32 = mode_ == EP2D_MODE_SPLIT;
       if (multiIter_) {
         auto segsOf = [&](int4* out) {
           if (ipl_ == 2) return march2_segments(nX, nY, marchRows_, 0, out);
@@ -342,46 +347,162 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
           return chain_segments(ipl_, nX, nY, marchRows_, 0, out, stageWaves_);
         };
         const int raw = segsOf(nullptr);
-        const int2 dims = make_int2(nX, nY);
         const bool ordered = ipl_ >= 3 && !wide_;
-        const int res = ordered ? chain_resident(ipl_, stageWaves_, mode_ == EP2D_MODE_SPLIT) : 0;
-        nSegs2_ = ordered ? chain_work_order(nullptr, raw, stageWaves_, &dims, res, nullptr) : raw;
-        std::vector<int4> s2((size_t)nSegs2_);
+        const int res = ordered ? chain_resident(ipl_, stageWaves_, f32) : 0;
+        s2.resize((size_t)(ordered ? chain_work_order(nullptr, raw, stageWaves_, &dims, res, nullptr)
+                                   : raw));
         segsOf(s2.data());
         if (ordered) chain_work_order(s2.data(), raw, stageWaves_, &dims, res, s2.data());
-        dSegs2_ = (int4*)alloc(s2.size() * sizeof(int4));
-        EP2D_HIP(hipMemcpyAsync(dSegs2_, s2.data(), s2.size() * sizeof(int4),
-                                hipMemcpyHostToDevice, stream_));
-        EP2D_HIP(hipStreamSynchronize(stream_));
       }
       if (ipl_ >= 3) {
-        std::vector<int4> c3, c2((size_t)march2_segments(nX, nY, 26, 0, nullptr));
-        march2_segments(nX, nY, 26, 0, c2.data());
+        // closing launches of 26 and 42 rows, of fewer on a small grid
+        const int r2 = tileSingles_ ? std::min(26, marchRows_) : 26;
+        const int r3 = tileSingles_ ? std::min(42, marchRows_) : 42;
+        c2.resize((size_t)march2_segments(nX, nY, r2, 0, nullptr));
+        march2_segments(nX, nY, r2, 0, c2.data());
         if (ipl_ == 4) {
-          const int raw = chain_segments(3, nX, nY, 42, 0, nullptr, 1);
-          const int2 dims = make_int2(nX, nY);
-          const int res = chain_resident(3, 1, mode_ == EP2D_MODE_SPLIT);
+          const int raw = chain_segments(3, nX, nY, r3, 0, nullptr, 1);
+          const int res = chain_resident(3, 1, f32);
           c3.resize((size_t)chain_work_order(nullptr, raw, 1, &dims, res, nullptr));
-          chain_segments(3, nX, nY, 42, 0, c3.data(), 1);
+          chain_segments(3, nX, nY, r3, 0, c3.data(), 1);
           chain_work_order(c3.data(), raw, 1, &dims, res, c3.data());
         }
-        nSegsC3_ = (int)c3.size();
-        nSegsC2_ = (int)c2.size();
-        if (nSegsC3_ > 0) {
-          dSegsC3_ = (int4*)alloc(c3.size() * sizeof(int4));
-          EP2D_HIP(hipMemcpyAsync(dSegsC3_, c3.data(), c3.size() * sizeof(int4),
-                                  hipMemcpyHostToDevice, stream_));
-        }
-        dSegsC2_ = (int4*)alloc(c2.size() * sizeof(int4));
-        EP2D_HIP(hipMemcpyAsync(dSegsC2_, c2.data(), c2.size() * sizeof(int4),
-                                hipMemcpyHostToDevice, stream_));
       }
-      EP2D_HIP(hipStreamSynchronize(stream_));
+      nSegs2_ = (int)s2.size();
+      nSegsC3_ = (int)c3.size();
+      nSegsC2_ = (int)c2.size();
+      std::vector<ResTile> tiles;
+      if (autoShape && !pool_) planResident(tiles);
+      // every table in one block, with one copy
+      RveDev rd = r_;
+      rd.cur = 0;
+      const std::pair<const void*, size_t> parts[] = {
+          {&rd, sizeof(rd)},
+          {segs.data(), segs.size() * sizeof(int4)},
+          {s2.data(), s2.size() * sizeof(int4)},
+          {c3.data(), c3.size() * sizeof(int4)},
+          {c2.data(), c2.size() * sizeof(int4)},
+          {tiles.data(), tiles.size() * sizeof(ResTile)}};
+      size_t at[7] = {0};
+      for (int k = 0; k < 6; k++) at[k + 1] = at[k] + (parts[k].second + 255) / 256 * 256;
+      std::vector<char> host(at[6], 0);
+      for (int k = 0; k < 6; k++)
+        if (parts[k].second) std::memcpy(host.data() + at[k], parts[k].first, parts[k].second);
+      // (after the tables: the record and exchange buffer of resident runs)
+      const size_t resBytes = resTiles_ ? 256 + 2 * (size_t)resXpar_ : 0;
+      char* blk = (char*)alloc(at[6] + resBytes);
+      dRve_ = (RveDev*)blk;
+      dSegs_ = (int4*)(blk + at[1]);
+      dSegs2_ = (int4*)(blk + at[2]);
+      dSegsC3_ = (int4*)(blk + at[3]);
+      dSegsC2_ = (int4*)(blk + at[4]);
+      dResTiles_ = (ResTile*)(blk + at[5]);
+      if (resTiles_) {
+        dResCtl_ = (ResCtl*)(blk + at[6]);
+        dXch_ = blk + at[6] + 256;
+        launch_fill((double*)(blk + at[6]), resBytes / 8, 0.0, stream_);
+      }
+      h2d(blk, host.data(), host.size());
     }
   }
   EP2D_HIP(hipStreamSynchronize(stream_));
 
   if (!logPath_.empty()) log_.open(logPath_, std::ios_base::app);   // :1607
+}
+
+// Shape of the resident runs of a handle on the automatic shape, and its tiles.
+void Solver::planResident(std::vector<ResTile>& tiles) {
+  if (nX_ < kResMinSide) return;
+  resRoom_ = (unsigned)resident_room(device_);
+  for (const ResShape& sh : resident_shapes(mode_)) {
+    size_t pairs = 0;
+    const int n = resident_tiles(sh, mode_, nX_, 0, 0, nullptr, &pairs);
+    const int cost = n > 0 ? resident_cost(sh, mode_) : 0;
+    if (cost == 0 || (size_t)n * (size_t)cost > resRoom_ || pairs * 16 > 0x7fffffffu) continue;
+    tiles.resize((size_t)n);
+    resident_tiles(sh, mode_, nX_, 0, 0, tiles.data(), nullptr);
+    resShape_ = sh;
+    resCost_ = (unsigned)cost;
+    resXpar_ = (unsigned)((pairs * 16 + 255) / 256 * 256);
+    resTiles_ = n;
+    hResTold_ = (unsigned*)(hMax_ + 3);  // the word past the residual's three
+    return;
+  }
+}
+
+// Whether n iterations run resident now: a handle with such a shape, and enough
+// iterations to pay for the start (the tiles' arrival and the loads of the
+// state take about ten microseconds).
+bool Solver::residentFits(long n) {
+  if (resTiles_ == 0 || n < kResMinIters || stress64_) return false;
+  if (resSkip_ > 0) {
+    resSkip_--;
+    return false;
+  }
+  return true;
+}
+
+void Solver::launchResidentRun(long n) {
+  const bool timed = sampleEvery_ > 0 && (launchCount_ % sampleEvery_) == 0;
+  std::pair<hipEvent_t, hipEvent_t> ev{};
+  if (timed) ev = takeTimingEvents();
+  if (resTag_ > 0xffffffffu - (unsigned)n) {
+    launch_fill((double*)dXch_, 2 * (size_t)resXpar_ / 8, 0.0, stream_);
+    resTag_ = 0;
+  }
+  ResLaunch a{};
+  a.mode = mode_;
+  a.shape = resShape_;
+  a.rves = dRve_;
+  a.list = dResTiles_;
+  a.tiles = resTiles_;
+  a.parity = cur_;
+  a.vpar = vIdx_;
+  a.iters = (int)n;
+  a.xch = dXch_;
+  a.xpar = resXpar_;
+  a.tag0 = resTag_;
+  a.ctl = dResCtl_;
+  a.cost = resCost_;
+  a.room = resRoom_;
+  a.told = hResTold_;
+  *hResTold_ = 0;
+  launch_resident(a, stream_, timed ? ev.first : nullptr, timed ? ev.second : nullptr);
+  resTag_ += (unsigned)n;
+  resPending_ = n;
+  cur_ ^= 1;
+  stressStale_ = true;
+  if (timed) {
+    pending_.push_back(ev);
+    pendingIters_.push_back((int)n);
+    if (pending_.size() >= 256) resolveTiming(false);
+  }
+  launchCount_++;
+}
+
+// Outcome of the last resident run, the stream being idle: true when there
+// was none or it ran; else its iterations have been launched on the other
+// kernels.
+bool Solver::settled() {
+  if (resPending_ == 0) return true;
+  const long n = resPending_;
+  resPending_ = 0;
+  const unsigned how = *hResTold_;
+  if (how == kResGo) return true;
+  if (how != kResNoRoom && how != kResLate)
+    throw HipError("a resident run lost a wait for a neighbouring tile");
+  if (how == kResLate) resSkip_ = 256;
+  cur_ ^= 1;
+  iterateLaunches(n);
+  return false;
+}
+
+// Before anything that uses the state: a resident run's outcome is known.
+void Solver::settle() {
+  if (resPending_ == 0) return;
+  EP2D_HIP(hipSetDevice(device_));
+  EP2D_HIP(hipStreamSynchronize(stream_));
+  settled();
 }
 
 Solver::~Solver() { release(); }
@@ -557,7 +678,7 @@ void Solver::launchIteration() {
     if (stress64_)
       launch_fused(r_, cur_, kModeSplitStress64, plastic, fplan64_, stream_,
                    timed ? ev.first : nullptr, timed ? ev.second : nullptr);
-    else if (marchRows_ > 0)
+    else if (marchRows_ > 0 && !tileSingles_)
       launch_march(dRve_, dSegs_, nSegs_, mode_, cur_, vIdx_, stream_,
                    timed ? ev.first : nullptr, timed ? ev.second : nullptr);
     else
@@ -632,6 +753,22 @@ int Solver::iterMode() const { return stress64_ ? kModeSplitStress64 : mode_; }
 
 void Solver::iterate(long n) {
   EP2D_HIP(hipSetDevice(device_));
+  settle();
+  if (residentFits(n)) {
+    // (a launch of a second at most, which other handles' work may wait for)
+    constexpr long kMost = 1L << 16;
+    for (; n > kMost; n -= kMost) {
+      launchResidentRun(kMost);
+      settle();
+    }
+    if (n >= kResMinIters) launchResidentRun(n);
+    else iterateLaunches(n);
+    return;
+  }
+  iterateLaunches(n);
+}
+
+void Solver::iterateLaunches(long n) {
   if (!multiIter_ || (stress64_ && !multi64())) {
     for (long k = 0; k < n; k++) launchIteration();
     return;
@@ -689,6 +826,7 @@ void Solver::resolveTiming(bool all) {
 }
 
 void Solver::setTiming(long sampleEvery) {
+  settle();
   resolveTiming(true);
   sampleEvery_ = sampleEvery < 0 ? 0 : sampleEvery;
   timedMs_ = 0.0;
@@ -697,6 +835,7 @@ void Solver::setTiming(long sampleEvery) {
 }
 
 void Solver::getTiming(double* avgMs, long* samples, const char** name) {
+  settle();
   resolveTiming(true);
   if (avgMs) *avgMs = timedSamples_ ? timedMs_ / timedSamples_ : 0.0;
   if (samples) *samples = timedSamples_;
@@ -705,7 +844,12 @@ void Solver::getTiming(double* avgMs, long* samples, const char** name) {
     // the handle's destruction
     std::string& nm = timingName_;
     nm = fused_kernel_name(mode_);
-    if (marchRows_ > 0 && multiIter_)
+    if (resTiles_ > 0)
+      nm = std::string(mode_ == EP2D_MODE_SPLIT ? "k_resident<float, float, "
+                                                : "k_resident<double, double, ") +
+           std::to_string(resShape_.rows) + ", " + std::to_string(resShape_.every) + ", " +
+           std::to_string(resShape_.waves) + "> tiles=" + std::to_string(resTiles_) + " (per iteration)";
+    else if (marchRows_ > 0 && multiIter_)
       nm = (ipl_ == 2 ? std::string(mode_ == EP2D_MODE_SPLIT ? "k_march2p<float, float>"
                                                               : "k_march2p<double, double>")
             : wide_ ? "k_wide<" + std::to_string(ipl_) + ">"
@@ -726,12 +870,16 @@ void Solver::getTiming(double* avgMs, long* samples, const char** name) {
   }
 }
 
-void Solver::sync() { EP2D_HIP(hipStreamSynchronize(stream_)); }
+void Solver::sync() {
+  settle();
+  EP2D_HIP(hipStreamSynchronize(stream_));
+}
 
 // Stress fields as the reference holds them after the loop: the trial stress
 // of U^{n-1} after the return mapping (the fused schemes keep it on chip, so
 // it is recomputed here in FP64 from the previous displacement buffer).
 void Solver::ensureStress() {
+  settle();
   if (!stressStale_) return;
   const int prev = cur_ ^ 1;
   launch_plain_stress(r_, r_.Ux[prev], r_.Uy[prev], f_, stream_);
@@ -743,13 +891,18 @@ void Solver::ensureStress() {
 }
 
 void Solver::applyAffine(double dUxdx, double dUydy, double dUxdy, double dUydx) {
+  settle();
   launch_affine(r_.Ux[cur_], r_.Uy[cur_], nX_, nY_, dX_, dY_, dUxdx, dUydy, dUxdy, dUydx, stream_);
 }
 
 // EffPlast2D.cu:407-412 (step-level entry point).
 double Solver::residual(const double e[3], long* nonfinite) {
-  launch_maxabs(r_, mode_ == EP2D_MODE_SPLIT, dMax_, stream_);
-  d2h(hMax_, dMax_, 3);
+  // (a resident run that did not start is made up for, and the residual taken
+  // again)
+  do {
+    launch_maxabs(r_, mode_ == EP2D_MODE_SPLIT, dMax_, stream_);
+    d2h(hMax_, dMax_, 3);
+  } while (!settled());
   double mx, my;
   std::memcpy(&mx, &hMax_[0], 8);
   std::memcpy(&my, &hMax_[1], 8);
@@ -864,6 +1017,7 @@ double find_max_abs_signed(const double* v, int n) {   // EffPlast2D.cu:814-822
 // Pore-edge hole area, EffPlast2D.cu:514-620.  Uses the values gathered by
 // the last boundary() call (same state).
 void Solver::holeArea(ep2d_record& r) {
+  settle();
   if (!samplesValid_)
     throw StatusError(EP2D_ERR_GEOMETRY,
                       "pore-edge sample window outside the grid (pores too large or too close "
@@ -946,6 +1100,7 @@ void Solver::jobBegin(int kind, double initLoadValue, const double loadType[3], 
 
 // Start of a time step (EffPlast2D.cu:312-384): banner, macro strain, affine U increment.
 void Solver::tsBegin() {
+  settle();
   const TaskPlan& tp = plan_[task_];
   const int step = (int)task_;
   if (tstep_ == 0) {
@@ -1231,8 +1386,10 @@ void Solver::runJob(ep2d_result* out) {
       iterate(c);
       tsDone_ += c;
       if (tsAtCheck()) {
-        tsCheckLaunch();
-        EP2D_HIP(hipStreamSynchronize(stream_));
+        do {
+          tsCheckLaunch();
+          EP2D_HIP(hipStreamSynchronize(stream_));
+        } while (!settled());
         tsCheckFinish();
       }
     }
@@ -1382,6 +1539,7 @@ void Solver::getField(int field, double* host, size_t count) {
   const size_t N = (size_t)m * n;
   if (count < N) throw ArgError("host buffer too small for field");
   EP2D_HIP(hipSetDevice(device_));
+  settle();
   switch (field) {
     case EP2D_FIELD_P: ensureStress(); d2h(host, f_.P, N); return;
     case EP2D_FIELD_TAUXX: ensureStress(); d2h(host, f_.tauXX, N); return;
@@ -1418,6 +1576,7 @@ void Solver::getField(int field, double* host, size_t count) {
 // first); the stream is synchronised, so the buffer is ready for any stream.
 const void* Solver::fieldDevice(int field) {
   EP2D_HIP(hipSetDevice(device_));
+  settle();
   const void* p = nullptr;
   switch (field) {
     case EP2D_FIELD_P: ensureStress(); p = f_.P; break;
@@ -1443,6 +1602,7 @@ void Solver::setField(int field, const double* host, size_t count) {
   const size_t N = (size_t)m * n;
   if (count < N) throw ArgError("host buffer too small for field");
   EP2D_HIP(hipSetDevice(device_));
+  settle();
   switch (field) {
     case EP2D_FIELD_UX: h2d(r_.Ux[cur_], host, N); return;
     case EP2D_FIELD_UY: h2d(r_.Uy[cur_], host, N); return;

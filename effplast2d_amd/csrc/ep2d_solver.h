@@ -183,8 +183,27 @@ class Solver {
   int nSegsC3_ = 0, nSegsC2_ = 0;
   int4* dSegsC3_ = nullptr;
   int4* dSegsC2_ = nullptr;
+  bool tileSingles_ = false;        // single iterations on the tile kernel
   int vIdx_ = 0;                    // velocity buffer holding the current V
   void flipV();                     // the other velocity buffer becomes current
+  // resident runs (ep2d_resident.hip): the shape of this grid (resTiles_ 0:
+  // none), its tile list, exchange buffer and launch record in one block, and
+  // the run whose outcome has not been read yet (its iterations, 0: none)
+  int resTiles_ = 0;
+  ResShape resShape_;
+  unsigned resCost_ = 0, resRoom_ = 0, resTag_ = 0, resXpar_ = 0;
+  ResTile* dResTiles_ = nullptr;
+  char* dXch_ = nullptr;
+  ResCtl* dResCtl_ = nullptr;
+  unsigned* hResTold_ = nullptr;
+  long resPending_ = 0;
+  int resSkip_ = 0;                 // runs to take the other kernels after a late start
+  void planResident(std::vector<ResTile>& tiles);
+  bool residentFits(long n);
+  void launchResidentRun(long n);
+  bool settled();                   // after the stream is synchronised
+  void settle();
+  void iterateLaunches(long n);
   std::pair<hipEvent_t, hipEvent_t> takeTimingEvents();
   void launchMulti(int q);         // ipl_ iterations, q-th such launch of a run
   void launchClose(int ns, int q);  // ns = 3 or 2 iterations closing a run
