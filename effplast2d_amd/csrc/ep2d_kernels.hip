@@ -555,16 +555,6 @@ struct Fused {
   }
 };
 
-// Block -> tile map.  Workgroups are dispatched round-robin over the 8 XCDs
-// (block b to XCD b % 8), so XCD x receives its blocks as a contiguous run of
-// the tile list: x*q + min(x, r) + b/8 with q = nb/8, r = nb%8 (the first r
-// XCDs take one more).  A tile and its neighbours, which share halo rows,
-// then mostly run on the same XCD and share its L2.
-__device__ __forceinline__ int tile_of_block(int b, int nb) {
-  const int x = b & 7, q = nb >> 3, r = nb & 7;
-  return x * q + min(x, r) + (b >> 3);
-}
-
 template <typename CT, typename VT, bool PLASTIC, int TY, int NW>
 __global__ __launch_bounds__(64 * NW) void k_fused(RveDev r, int cur, int ntx, int ntiles) {
   using F = Fused<CT, VT, PLASTIC, TY, NW>;
@@ -982,103 +972,9 @@ __global__ __launch_bounds__(256) void k_march(const RveDev* __restrict__ rves,
   else March<CT, VT>::template run<true>(r, cur, vpar, s, j0, j1, gt[wave]);
 }
 
-// Stage A's inputs in a two-iteration segment: the first rows (start) and,
-// for step t, Ux row t+1, Uy row t+2, mask row t+1 and V row t of the state in
-// HBM, through buffer resources (the lane's byte offset fixed, the row's in an
-// SGPR).  Interior segments clamp rows to the segment's last step tEnd.  Edge
-// segments bound each resource to its field: lanes outside the field's
-// columns carry the offset kOob, and a row outside the field reads through a
-// resource of bound 0, so every such load returns 0 without a branch.
-template <typename CT, typename VT, bool EX, bool EY = EX, bool CLEAN = false>
-struct StageInput {
-  static constexpr bool EDGE = EX || EY;
-  using Ld = typename March<CT, VT>::Ld;
-  const double* Uxi;
-  const double* Uyi;
-  const VT* Vxi;
-  const VT* Vyi;
-  const unsigned char* mask;
-  int nX, nY, sx, i, tEnd;
-  unsigned o8, oV;
-  __amdgpu_buffer_rsrc_t bUx, bUy, bVx, bVy, bM;
-  // edge segments: lane offsets with the column test folded in (Ux columns
-  // 0..nX, the others 0..nX-1; V is read for columns 0..nX-1 only)
-  unsigned oUx, oC8, oM, oVc;
-
-  __device__ __forceinline__ StageInput(const RveDev& r, int cur, int vpar, int col, int tEnd_)
-      : Uxi(r.Ux[cur]), Uyi(r.Uy[cur]),
-        Vxi(static_cast<const VT*>(vpar ? r.Vx2 : r.Vx)),
-        Vyi(static_cast<const VT*>(vpar ? r.Vy2 : r.Vy)), mask(r.mask), nX(r.nX), nY(r.nY),
-        sx(r.nX + 1), i(col), tEnd(tEnd_), o8((unsigned)col * 8u),
-        oV((unsigned)col * (unsigned)sizeof(VT)) {
-    if (!EDGE) {
-      bUx = brsrc(Uxi);
-      bUy = brsrc(Uyi);
-      bVx = brsrc(Vxi);
-      bVy = brsrc(Vyi);
-      bM = brsrc(mask);
-    } else {
-      const unsigned ux = (unsigned)nY * (unsigned)sx, uy = (unsigned)(nY + 1) * (unsigned)nX;
-      bUx = brsrc_n(Uxi, ux * 8u);
-      bUy = brsrc_n(Uyi, uy * 8u);
-      bVx = brsrc_n(Vxi, ux * (unsigned)sizeof(VT));
-      bVy = brsrc_n(Vyi, uy * (unsigned)sizeof(VT));
-      bM = brsrc_n(mask, (unsigned)nY * (unsigned)nX);
-      const bool cx = col >= 0 && col <= nX, cc = col >= 0 && col < nX;
-      oUx = cx ? o8 : kOob;
-      oC8 = cc ? o8 : kOob;
-      oM = cc ? (unsigned)col : kOob;
-      oVc = cc ? oV : kOob;
-    }
-  }
-
-  // Ux row jb, Uy row jb+1, mask row jb into the stage
-  __device__ __forceinline__ void start(MarchStage<CT, VT, EX, EY, CLEAN>& st, int jb) const {
-    double ux = 0.0, uy = 0.0;
-    unsigned m = 0;
-    const bool colC = !EDGE || (i >= 0 && i < nX);
-    if (!EDGE) {
-      ux = gld(Uxi, (unsigned)(jb * sx + i));
-      uy = gld(Uyi, (unsigned)((jb + 1) * nX + i));
-      if (!CLEAN) m = gld(mask, (unsigned)(jb * nX + i));
-    } else {
-      if (i >= 0 && i <= nX && jb >= 0 && jb < nY) ux = gld(Uxi, (unsigned)(jb * sx + i));
-      if (colC && jb + 1 >= 0 && jb + 1 <= nY) uy = gld(Uyi, (unsigned)((jb + 1) * nX + i));
-      if (!CLEAN && colC && jb >= 0 && jb < nY) m = gld(mask, (unsigned)(jb * nX + i));
-    }
-    st.start(ux, uy, m);
-  }
-
-  __device__ __forceinline__ Ld fetch(int t0) const {
-    const int t = EDGE ? t0 : min(t0, tEnd);
-    Ld d;
-    if (!EDGE) {
-      d.ux = bld<double>(bUx, o8, (unsigned)(t + 1) * (unsigned)sx * 8u);
-      d.uy = bld<double>(bUy, o8, (unsigned)(t + 2) * (unsigned)nX * 8u);
-      d.m = CLEAN ? 0u : bld<unsigned char>(bM, (unsigned)i, (unsigned)(t + 1) * (unsigned)nX);
-      d.vx = bld<VT>(bVx, oV, (unsigned)t * (unsigned)sx * (unsigned)sizeof(VT));
-      d.vy = bld<VT>(bVy, oV, (unsigned)t * (unsigned)nX * (unsigned)sizeof(VT));
-    } else {
-      // rows outside a field read through a resource of bound 0 (the row
-      // tests are uniform: scalar selects); the row offset is then 0
-      const __amdgpu_buffer_rsrc_t none = brsrc_n(Uxi, 0u);
-      const bool r1 = t + 1 >= 0 && t + 1 < nY, r2 = t + 2 >= 0 && t + 2 <= nY,
-                 r0 = t >= 0 && t < nY;
-      const unsigned s1 = r1 ? (unsigned)(t + 1) : 0u, s2 = r2 ? (unsigned)(t + 2) : 0u,
-                     s0 = r0 ? (unsigned)t : 0u;
-      d.ux = bld<double>(r1 ? bUx : none, oUx, s1 * (unsigned)sx * 8u);
-      d.uy = bld<double>(r2 ? bUy : none, oC8, s2 * (unsigned)nX * 8u);
-      d.m = CLEAN ? 0u : bld<unsigned char>(r1 ? bM : none, oM, s1 * (unsigned)nX);
-      d.vx = bld<VT>(r0 ? bVx : none, oVc, s0 * (unsigned)sx * (unsigned)sizeof(VT));
-      d.vy = bld<VT>(r0 ? bVy : none, oVc, s0 * (unsigned)nX * (unsigned)sizeof(VT));
-    }
-    return d;
-  }
-};
-
 template <typename CT, typename VT, bool EDGE>
 __device__ __forceinline__ void march2_run(const RveDev& r, int cur, int vpar, int s, int j0,
-                                           int j1, const CT* gt) {
+                                           int j1, const VertMod<CT>* gt) {
   using M = March<CT, VT>;
   using Ld = typename M::Ld;
   const int nX = r.nX, nY = r.nY, sx = nX + 1;
@@ -1104,7 +1000,8 @@ __device__ __forceinline__ void march2_run(const RveDev& r, int cur, int vpar, i
   unsigned mh1 = 0, mh2 = 0;
   auto fetch = [&](int t) { return in.fetch(t); };
   auto body = [&](const int t, const Ld& ld) {
-    const auto oA = A.step(t, ld.ux, ld.uy, ld.m, (CT)ld.vx, (CT)ld.vy);
+    const unsigned m = stage_mask(ld.m);
+    const auto oA = A.step(t, ld.ux, ld.uy, m, (CT)ld.vx, (CT)ld.vy);
     if (t == jbB + 1) B.start(h1ux, oA.uy, mh2);  // Ux' row jbB, Uy' row jbB+1, mask row jbB
     if (t >= jbB + 2) {
       const int j = t - 2;
@@ -1128,7 +1025,7 @@ __device__ __forceinline__ void march2_run(const RveDev& r, int cur, int vpar, i
     h1vx = oA.vx;
     h1vy = oA.vy;
     mh2 = mh1;
-    mh1 = ld.m;
+    mh1 = m;
   };
   Ld P = fetch(jbA);
   for (int t = jbA; t <= tEnd; t += 2) {
@@ -1144,7 +1041,7 @@ template <typename CT, typename VT>
 __global__ __launch_bounds__(256) void k_march2(const RveDev* __restrict__ rves,
                                                 const int4* __restrict__ segs, int nsegs,
                                                 int parity, int vpar) {
-  __shared__ CT gt[4][16];
+  __shared__ VertMod<CT> gt[4][16];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int b = tile_of_block(blockIdx.x, gridDim.x);
@@ -1152,7 +1049,7 @@ __global__ __launch_bounds__(256) void k_march2(const RveDev* __restrict__ rves,
   if (k >= nsegs) return;
   const int4 sg = segs[k];
   const RveDev& r = rves[sg.x];
-  if (lane < 16) gt[wave][lane] = (CT)r.gtab[lane];
+  if (lane < 16) gt[wave][lane].g = (CT)r.gtab[lane];
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's table is in LDS
   __builtin_amdgcn_wave_barrier();
   const int cur = parity ^ r.cur;
@@ -1190,7 +1087,7 @@ struct RowRing {
 // a slot and the barrier after each step orders a write before its reads.
 template <typename CT, typename VT, bool EDGE>
 __device__ __forceinline__ void march2p_run(const RveDev& r, int cur, int vpar, int s, int j0,
-                                            int j1, const CT* gt, bool stageB,
+                                            int j1, const VertMod<CT>* gt, bool stageB,
                                             RowRing<CT>& ring, int nSteps) {
   using M = March<CT, VT>;
   using Ld = typename M::Ld;
@@ -1207,12 +1104,13 @@ __device__ __forceinline__ void march2p_run(const RveDev& r, int cur, int vpar, 
     auto stepA = [&](int q, const Ld& ld, int sl) {
       const int t = jbA + q;
       if (t <= tEnd) {
-        const auto o = st.step(t, ld.ux, ld.uy, ld.m, (CT)ld.vx, (CT)ld.vy);
+        const unsigned m = stage_mask(ld.m);
+        const auto o = st.step(t, ld.ux, ld.uy, m, (CT)ld.vx, (CT)ld.vy);
         ring.ux[sl][L] = o.ux;
         ring.uy[sl][L] = o.uy;
         ring.vx[sl][L] = o.vx;
         ring.vy[sl][L] = o.vy;
-        ring.m[sl][L] = ld.m;
+        ring.m[sl][L] = m;
       }
       lds_barrier();
     };
@@ -1286,7 +1184,7 @@ template <typename CT, typename VT>
 __global__ __launch_bounds__(256) void k_march2p(const RveDev* __restrict__ rves,
                                                  const int4* __restrict__ segs, int nsegs,
                                                  int parity, int vpar) {
-  __shared__ CT gt[4][16];
+  __shared__ VertMod<CT> gt[4][16];
   __shared__ RowRing<CT> ring[2];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -1307,7 +1205,7 @@ __global__ __launch_bounds__(256) void k_march2p(const RveDev* __restrict__ rves
   }
   const int4 sg = segs[k];
   const RveDev& r = rves[sg.x];
-  if (lane < 16) gt[wave][lane] = (CT)r.gtab[lane];
+  if (lane < 16) gt[wave][lane].g = (CT)r.gtab[lane];
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's table is in LDS
   __builtin_amdgcn_wave_barrier();
   const int cur = parity ^ r.cur;
@@ -1335,24 +1233,6 @@ __global__ void k_mask_map(const unsigned char* __restrict__ mask, int nX, int n
   map[b] = any ? 1 : 0;
 }
 
-// Whether the mask is 0 over rows [jlo, jhi] and columns [ilo, ihi] (clipped
-// to the grid), from the block map; the same answer in every lane.
-__device__ __forceinline__ bool mask_clear(const RveDev& r, int ilo, int ihi, int jlo, int jhi) {
-  ilo = max(ilo, 0);
-  jlo = max(jlo, 0);
-  ihi = min(ihi, r.nX - 1);
-  jhi = min(jhi, r.nY - 1);
-  if (ilo > ihi || jlo > jhi) return true;
-  const int bx0 = ilo / kMapCols, bx1 = ihi / kMapCols;
-  const int by0 = jlo / kMapRows, by1 = jhi / kMapRows;
-  const int nbx = (r.nX + kMapCols - 1) / kMapCols;
-  const int w = bx1 - bx0 + 1, n = w * (by1 - by0 + 1);
-  unsigned any = 0;
-  for (int q = (int)(threadIdx.x & 63); q < n; q += 64)
-    any |= r.mmap[(by0 + q / w) * nbx + bx0 + q % w];
-  return !__any(any != 0);
-}
-
 // NS iterations per launch on a chain of NS waves (one workgroup).  Stage 0
 // reads the state from HBM and runs the first iteration, stage k the (k+1)-th
 // from the rows of stage k-1, and the last stage writes the result.  Each
@@ -1377,21 +1257,25 @@ __device__ __forceinline__ bool mask_clear(const RveDev& r, int ilo, int ihi, in
 // and writes the entries it computes exactly (lanes 2..61, the union's outer
 // lanes 0, 1 and 62, 63 included), each position once.  Only the union's
 // outer edges lose two columns per stage: strips of 60W+4-4NS outputs.
-template <typename CT, typename VT, bool EX, bool EY, bool CLEAN, int NS, int W>
+template <typename CT, typename VT, bool EX, bool EY, bool CLEAN, int PL, int NS, int W>
 __device__ __forceinline__ void chain_run(const RveDev& r, int cur, int vpar, int s, int j0,
-                                          int j1, const CT* gt, int role, int c,
+                                          int j1, const VertMod<CT>* gt, int role, int c,
                                           RowRing<CT, W>* ring, int nSteps) {
   constexpr bool EDGE = EX || EY;
   constexpr int UW = 60 * W + 4;  // columns of the union of a stage's waves
   using M = March<CT, VT>;
   using Ld = typename M::Ld;
-  using Stage = MarchStage<CT, VT, EX, EY, CLEAN>;
+  using Stage = MarchStage<CT, VT, EX, EY, CLEAN, PL>;
   const int nX = r.nX, nY = r.nY, sx = nX + 1;
   const int L = threadIdx.x & 63;
   const int P = W == 1 ? L : 60 * c + L;  // position in the union (and the ring row)
   const int i = s + P;
-  // the lanes whose outputs this wave hands on (each ring position once)
+  // the lanes whose outputs this wave hands on (each ring position once); the
+  // others write past the union, where nothing is read, so a step has no
+  // branch over its lanes
   const bool wl = W == 1 || ((c == 0 || L >= 2) && (c == W - 1 || L < 62));
+  const int Pw = wl ? P : P + 64;
+  static_assert(W <= 2, "positions 124 .. 127 lie past the union");
   const int jbA = j0 - 2 * NS, tEnd = j1 + 2 * NS - 3;
   Stage st;
   st.setup(r, gt, i);
@@ -1413,14 +1297,13 @@ __device__ __forceinline__ void chain_run(const RveDev& r, int cur, int vpar, in
     in.start(st, jbA);
     const int nAct = tEnd - jbA + 1;
     auto stepA = [&](int q, const Ld& ld, auto sl) {
-      const auto o = st.step(jbA + q, ld.ux, ld.uy, ld.m, (CT)ld.vx, (CT)ld.vy);
-      if (wl) {
-        out.ux[sl][P] = o.ux;
-        out.uy[sl][P] = o.uy;
-        out.vx[sl][P] = o.vx;
-        out.vy[sl][P] = o.vy;
-        if (!CLEAN) out.m[sl][P] = ld.m;
-      }
+      const unsigned m = CLEAN ? 0u : stage_mask(ld.m);
+      const auto o = st.step(jbA + q, ld.ux, ld.uy, m, (CT)ld.vx, (CT)ld.vy);
+      out.ux[sl][Pw] = o.ux;
+      out.uy[sl][Pw] = o.uy;
+      out.vx[sl][Pw] = o.vx;
+      out.vy[sl][Pw] = o.vy;
+      if (!CLEAN) out.m[sl][Pw] = m;
       lds_barrier();
     };
     Ld P = in.fetch(jbA), Q;
@@ -1463,17 +1346,19 @@ __device__ __forceinline__ void chain_run(const RveDev& r, int cur, int vpar, in
     VT* Vxo = static_cast<VT*>(vpar ? r.Vx : r.Vx2);
     VT* Vyo = static_cast<VT*>(vpar ? r.Vy : r.Vy2);
     const bool outLane = wl && P >= 2 * NS && P < UW - 2 * NS && (!EX || i < nX);
-    const unsigned o8 = (unsigned)i * 8u, oV = (unsigned)i * (unsigned)sizeof(VT);
-    // edge segments bound the V resources to their fields: a lane whose V
-    // ComputeDisp leaves alone stores at kOob, which the hardware drops
-    const unsigned vxb = (unsigned)nY * (unsigned)sx * (unsigned)sizeof(VT),
-                   vyb = (unsigned)(nY + 1) * (unsigned)nX * (unsigned)sizeof(VT);
-    const __amdgpu_buffer_rsrc_t bUx = brsrc(Uxo), bUy = brsrc(Uyo),
-                                 bVx = EDGE ? brsrc_n(Vxo, vxb) : brsrc(Vxo),
-                                 bVy = EDGE ? brsrc_n(Vyo, vyb) : brsrc(Vyo);
+    // the resources are bounded to their fields: the hardware drops a store at
+    // kOob, where lanes without output (interior segments) and those whose V
+    // ComputeDisp leaves alone (edge segments) point
+    const bool st8 = EDGE || outLane;
+    const unsigned o8 = st8 ? (unsigned)i * 8u : kOob,
+                   oV = st8 ? (unsigned)i * (unsigned)sizeof(VT) : kOob;
+    const unsigned nx = (unsigned)nY * (unsigned)sx, ny = (unsigned)(nY + 1) * (unsigned)nX;
+    const __amdgpu_buffer_rsrc_t bUx = brsrc_n(Uxo, nx * 8u), bUy = brsrc_n(Uyo, ny * 8u),
+                                 bVx = brsrc_n(Vxo, nx * (unsigned)sizeof(VT)),
+                                 bVy = brsrc_n(Vyo, ny * (unsigned)sizeof(VT));
     // step q reads Ux' of row j+1 (slot q-2), Uy' of row j+2 (slot q-1), V'
     // of row j and mask row j+1 (slot q-3); a middle stage writes slot q
-    auto stepK = [&](int q, auto ph) {
+    auto stepK = [&](int q, auto ph, auto store) {
       constexpr int s1 = (ph + 3) & 3, s2 = (ph + 2) & 3, s3 = (ph + 1) & 3;  // q-1, q-2, q-3
       const int j = jbA + q - lag;
       const double uxn = in.ux[s2][P], uynn = in.uy[s1][P];
@@ -1487,14 +1372,14 @@ __device__ __forceinline__ void chain_run(const RveDev& r, int cur, int vpar, in
                                       vxi, vyi)
                            : st.step(j, uxn, uynn, mn, vxi, vyi);
       if constexpr (!last) {
-        if (wl) {
-          out.ux[ph][P] = o.ux;
-          out.uy[ph][P] = o.uy;
-          out.vx[ph][P] = o.vx;
-          out.vy[ph][P] = o.vy;
-          if (!CLEAN) out.m[ph][P] = mn;
-        }
-      } else if (j >= j0 && outLane) {
+        out.ux[ph][Pw] = o.ux;
+        out.uy[ph][Pw] = o.uy;
+        out.vx[ph][Pw] = o.vx;
+        out.vy[ph][Pw] = o.vy;
+        if (!CLEAN) out.m[ph][Pw] = mn;
+      } else if (!store.value) {
+        // a row above the segment's
+      } else if (!EDGE || outLane) {
         const unsigned ovx = EDGE && !o.updX ? kOob : oV, ovy = EDGE && !o.updY ? kOob : oV;
         bst(bVx, ovx, (unsigned)j * (unsigned)sx * (unsigned)sizeof(VT), (VT)o.vx);
         bst(bVy, ovy, (unsigned)j * (unsigned)nX * (unsigned)sizeof(VT), (VT)o.vy);
@@ -1518,23 +1403,32 @@ __device__ __forceinline__ void chain_run(const RveDev& r, int cur, int vpar, in
         st.start(in.ux[s2][P], in.uy[s1][P], CLEAN ? 0u : in.m[s3][P]);
       lds_barrier();
     }
-    constexpr int P0 = (qStart + 1) & 3;
+    // the last stage's first two rows lie above the segment
+    constexpr int above = last ? 2 : 0;
+    using Yes = std::true_type;
+    using No = std::false_type;
+    constexpr int P0 = (qStart + 1 + above) & 3;
     using Q0 = std::integral_constant<int, P0>;
     using Q1 = std::integral_constant<int, (P0 + 1) & 3>;
     using Q2 = std::integral_constant<int, (P0 + 2) & 3>;
     using Q3 = std::integral_constant<int, (P0 + 3) & 3>;
     int q = qStart + 1;
+    if constexpr (above > 0) {
+      stepK(q, Q2{}, No{});
+      stepK(q + 1, Q3{}, No{});
+      q += 2;
+    }
     for (; q + 3 <= qLast; q += 4) {
-      stepK(q, Q0{});
-      stepK(q + 1, Q1{});
-      stepK(q + 2, Q2{});
-      stepK(q + 3, Q3{});
+      stepK(q, Q0{}, Yes{});
+      stepK(q + 1, Q1{}, Yes{});
+      stepK(q + 2, Q2{}, Yes{});
+      stepK(q + 3, Q3{}, Yes{});
     }
     if (q <= qLast) {
-      stepK(q, Q0{});
+      stepK(q, Q0{}, Yes{});
       if (q + 1 <= qLast) {
-        stepK(q + 1, Q1{});
-        if (q + 2 <= qLast) stepK(q + 2, Q2{});
+        stepK(q + 1, Q1{}, Yes{});
+        if (q + 2 <= qLast) stepK(q + 2, Q2{}, Yes{});
       }
     }
     idle(qLast + 1, nSteps);
@@ -1549,6 +1443,25 @@ __device__ __forceinline__ void chain_run(const RveDev& r, int cur, int vpar, in
   }
 }
 
+// What bounds it: with six waves to a SIMD, VALU issue -- 63 (split, plastic,
+// mask-free) instructions a row and wave, of which FP64 operations, conversions,
+// lane shifts and compares take four cycles and the others two if another
+// wave's fits beside -- and, where all segments run in one round, the slowest of
+// them, those at the left and right boundary.  Steps that got it here, us per
+// iteration before and after: 1024^2 split 7.2 -> 6.4, FP64 14.7 -> 13.7;
+// 2048^2 split 15.2 -> 14.1, FP64 41.4 -> 36.0; 4096^2 split 55.4 -> 54.0 (the
+// HBM traffic of 52 bytes a node and launch is 4 TB/s there), FP64 121.5 -> 115.0.
+// - Plastic and elastic interior segments have code of their own, and no lane
+//   branch: a step is one block of code up to the scaling.
+// - Carried sums (MarchStage) make a lane shift an operand of an addition.
+// - Mask bits select as widened words; vertex moduli are read at the byte
+//   offset the mask holds.
+// - Boundary columns and rows run the interior expressions on clamped blocks
+//   (they took 1.5 times an interior segment's time, now 1.2).
+// Two rows a step (half the barriers, four waves to a SIMD) took 6.9, 15.4, 16.4
+// and 37.8 us at 1024^2 and 2048^2, and loading stage 0's rows two or three
+// steps ahead the same as one.
+//
 // One segment per workgroup of NS x W waves (stage k on waves kW .. kW+W-1,
 // wave c of a stage on columns s+60c ..).  The split scheme's register
 // budget holds seven waves per SIMD (six with two waves per stage, where the
@@ -1561,7 +1474,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(CT) == 4 ? (W == 1 ? 7 : 6) : (W == 1 
                                                    const int4* __restrict__ segs, int nsegs,
                                                    int parity, int vpar) {
   constexpr int UW = 60 * W + 4;
-  __shared__ CT gt[NS * W][16];
+  __shared__ VertMod<CT> gt[16];
   __shared__ RowRing<CT, W> ring[NS - 1];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -1570,7 +1483,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(CT) == 4 ? (W == 1 ? 7 : 6) : (W == 1 
   if (k >= nsegs) return;  // the whole workgroup
   const int4 sg = segs[k];
   const RveDev& r = rves[sg.x];
-  if (lane < 16) gt[wave][lane] = (CT)r.gtab[lane];
+  if (lane < 16) gt[lane].g = (CT)r.gtab[lane];
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's table is in LDS
   __builtin_amdgcn_wave_barrier();
   const int cur = parity ^ r.cur;
@@ -1587,22 +1500,18 @@ __attribute__((amdgpu_waves_per_eu(sizeof(CT) == 4 ? (W == 1 ? 7 : 6) : (W == 1 
   const bool exAny = !(s >= 1 && s + UW - 1 <= r.nX - 2);
   const bool ey = !(j0 >= 2 * NS && j1 <= r.nY - (2 * NS - 1));
   const bool clean = !exAny && mask_clear(r, s, s + UW - 1, j0 - 2 * NS, j1 + 2 * NS - 2);
-  const CT* g = gt[wave];
-  if (ex)
-    chain_run<CT, VT, true, true, false, NS, W>(r, cur, vpar, s, j0, j1, g, role, c, ring,
-                                                nSteps);
-  else if (ey && clean)
-    chain_run<CT, VT, false, true, true, NS, W>(r, cur, vpar, s, j0, j1, g, role, c, ring,
-                                                nSteps);
-  else if (ey)
-    chain_run<CT, VT, false, true, false, NS, W>(r, cur, vpar, s, j0, j1, g, role, c, ring,
-                                                 nSteps);
-  else if (clean)
-    chain_run<CT, VT, false, false, true, NS, W>(r, cur, vpar, s, j0, j1, g, role, c, ring,
-                                                 nSteps);
-  else
-    chain_run<CT, VT, false, false, false, NS, W>(r, cur, vpar, s, j0, j1, g, role, c, ring,
-                                                  nSteps);
+  const VertMod<CT>* g = gt;
+  const bool pl = r.plastic != 0;
+#define EP2D_CHAIN(EX, EY, CLEAN, PL) \
+  chain_run<CT, VT, EX, EY, CLEAN, PL, NS, W>(r, cur, vpar, s, j0, j1, g, role, c, ring, nSteps)
+  if (ex) EP2D_CHAIN(true, true, false, -1);
+  else if (ey && clean) EP2D_CHAIN(false, true, true, -1);
+  else if (ey) EP2D_CHAIN(false, true, false, -1);
+  else if (clean && pl) EP2D_CHAIN(false, false, true, 1);
+  else if (clean) EP2D_CHAIN(false, false, true, 0);
+  else if (pl) EP2D_CHAIN(false, false, false, 1);
+  else EP2D_CHAIN(false, false, false, 0);
+#undef EP2D_CHAIN
 }
 
 // ---------------------------------------------------------------------------

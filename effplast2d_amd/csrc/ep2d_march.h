@@ -36,6 +36,16 @@ __device__ __forceinline__ void gst(T* base, unsigned idx, T v) {
   *(GT*)((GC*)base + idx * (unsigned)sizeof(T)) = v;
 }
 
+// Block -> tile map.  Workgroups are dispatched round-robin over the 8 XCDs
+// (block b to XCD b % 8), so XCD x receives its blocks as a contiguous run of
+// the tile list: x*q + min(x, r) + b/8 with q = nb/8, r = nb%8 (the first r
+// XCDs take one more).  A tile and its neighbours, which share halo rows,
+// then mostly run on the same XCD and share its L2.
+__device__ __forceinline__ int tile_of_block(int b, int nb) {
+  const int x = b & 7, q = nb >> 3, r = nb & 7;
+  return x * q + min(x, r) + (b >> 3);
+}
+
 // Raw buffer access for row marches: a resource (base in SGPRs; no range
 // limit, every access is in bounds by construction), a per-lane byte offset
 // fixed along the march and the row's byte offset, uniform, in an SGPR, so
@@ -499,25 +509,83 @@ struct March {
 // (segments whose mask bytes are all 0, chain kernels) read no mask: matrix
 // K and G, no pore zeroing and the vertex modulus of four matrix cells, which
 // is what the mask path computes from zero mask bytes.
-template <typename CT, typename VT, bool EX, bool EY = EX, bool CLEAN = false>
+//
+// PL 1 or 0 fixes whether the RVE is plastic (interior segments: a step is one
+// block of code up to the scaling); -1 reads it from the RVE.
+// The vertex moduli by class in LDS, eight bytes apart: the class bits of a mask
+// byte are the byte offset of its entry.
+template <typename CT>
+struct alignas(8) VertMod {
+  CT g;
+};
+template <typename CT>
+__device__ __forceinline__ CT vert_mod(const VertMod<CT>* gt, unsigned m) {
+  static_assert(M_VCLASS_SHIFT == 3 && sizeof(VertMod<CT>) == 8, "class bits as a byte offset");
+  return reinterpret_cast<const VertMod<CT>*>(reinterpret_cast<const char*>(gt) + (m & 0x78u))->g;
+}
+
+// Stages take the mask byte with its two zero bits inverted (1: the trial stress
+// stays), so that each bit, widened to a word, selects with one instruction
+// per 32 bits and without a compare.  (In assembly: the compiler would turn the
+// widened bit back into arithmetic.)
+__device__ __forceinline__ unsigned stage_mask(unsigned m) {
+  return m ^ (unsigned)(M_CELL_ZERO | M_VERT_ZERO);
+}
+template <int BIT>
+__device__ __forceinline__ unsigned mask_word(unsigned m) {
+  unsigned w;
+  asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(w) : "v"(m), "n"(__builtin_ctz(BIT)));
+  return w;
+}
+template <typename CT>
+__device__ __forceinline__ CT keep(unsigned w, CT a) {  // a, or 0 where w is 0
+  if constexpr (sizeof(CT) == 4) {
+    return __builtin_bit_cast(float, w & __builtin_bit_cast(unsigned, a));
+  } else {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, a);
+    return __builtin_bit_cast(double, (unsigned long long)(w & (unsigned)(b >> 32)) << 32 |
+                                          (w & (unsigned)b));
+  }
+}
+template <typename CT>
+__device__ __forceinline__ CT pick(unsigned w, CT yes, CT no) {
+  if constexpr (sizeof(CT) == 4) {
+    const unsigned a = __builtin_bit_cast(unsigned, yes), b = __builtin_bit_cast(unsigned, no);
+    return __builtin_bit_cast(float, (w & a) | (~w & b));
+  } else {
+    const unsigned long long a = __builtin_bit_cast(unsigned long long, yes),
+                             b = __builtin_bit_cast(unsigned long long, no);
+    const unsigned lo = (w & (unsigned)a) | (~w & (unsigned)b);
+    const unsigned hi = (w & (unsigned)(a >> 32)) | (~w & (unsigned)(b >> 32));
+    return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+  }
+}
+
+template <typename CT, typename VT, bool EX, bool EY = EX, bool CLEAN = false, int PL = -1>
 struct MarchStage {
   static constexpr bool EDGE = EX || EY;
   using M = March<CT, VT>;
   const RveDev* r;
-  const CT* gt;
+  const VertMod<CT>* gt;
   int nX, nY, i;
-  bool colC, colV, leftEdge, rightEdge, inX, plastic;
+  bool colC, colV, leftEdge, rightEdge, plastic;
   CT coh, c2lo, K0, Kp, G2_0, G2_p, P0, vdampX, vdampY, dTrho, g0;
   double dT;
   // grid steps held in registers: the stores of a step may alias the RVE
   // table, so values read from it would be read again after every store
   double dXd, dYd, rdXd, rdYd;
   CT rdXc, rdYc;
-  // carried rows: U rows j and j+1, mask row j, trial cells j (and j-1),
-  // trial vertices j-1 and j-2, corrected row j-1
+  // carried rows: U rows j and j+1, mask row j, trial cells j (and j-1) and
+  // their sums with the right neighbours, the sums of vertex row j-1 and of its
+  // 2x2 blocks, corrected row j-1 and the left neighbours of its shear.  The
+  // sums stand where the invariants' expressions begin, so a neighbour's value
+  // is needed in the step that computes it only (a lane shift there is an
+  // operand of the addition) and the trial stresses end with their step (the
+  // return mapping scales them in place).
   double ux_c, uxs_c, uy_c, uy_n;
   unsigned m_c;
-  CT tP_c, tXX_c, tYY_c, sXX_c, sYY_c, tP_p, tXX_p, tYY_p, tXY_p, tXY_pp, cP_p, cYY_p, cXY_p;
+  CT tP_c, tXX_c, tYY_c, hXX_c, hYY_c, tP_p, tXX_p, tYY_p, hXY_p, nXY_p, cP_p, cYY_p, cXY_p,
+      rXY_p;
 
   struct Out {
     double ux, uy;   // output U of row j at this lane's column
@@ -535,7 +603,7 @@ struct MarchStage {
           float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, (float)a)));
   }
 
-  __device__ __forceinline__ void setup(const RveDev& rr, const CT* g, int col) {
+  __device__ __forceinline__ void setup(const RveDev& rr, const VertMod<CT>* g, int col) {
     r = &rr;
     gt = g;
     nX = rr.nX;
@@ -543,7 +611,6 @@ struct MarchStage {
     i = col;
     colC = !EX || (i >= 0 && i < nX);
     colV = !EX || (i >= 0 && i < nX - 1);
-    inX = colC;
     leftEdge = EX && i == 0;
     rightEdge = EX && i == nX - 1;
     plastic = rr.plastic != 0;
@@ -589,10 +656,16 @@ struct MarchStage {
     uy_c = 0.0;
     uy_n = uy1;
     m_c = m;
-    tP_c = tXX_c = tYY_c = sXX_c = sYY_c = 0;
+    tP_c = tXX_c = tYY_c = hXX_c = hYY_c = 0;
     tP_p = tXX_p = tYY_p = 0;
-    tXY_p = tXY_pp = 0;
-    cP_p = cYY_p = cXY_p = 0;
+    hXY_p = nXY_p = 0;
+    cP_p = cYY_p = cXY_p = rXY_p = 0;
+  }
+
+  // FP32: the addition stays in the block of its shifted operand
+  static __device__ __forceinline__ CT here(CT a) {
+    if constexpr (sizeof(CT) == 4 && PL == 1) asm volatile("" : "+v"(a));
+    return a;
   }
 
   __device__ __forceinline__ Out step(const int j, const double ux_n, const double uy_nn,
@@ -609,8 +682,12 @@ struct MarchStage {
     // trial cell row j+1
     CT tP_n, tXX_n, tYY_n;
     {
-      const CT K = !CLEAN && (m_n & M_CELL_MAT) ? Kp : K0;
-      const CT G2 = !CLEAN && (m_n & M_CELL_MAT) ? G2_p : G2_0;
+      CT K = K0, G2 = G2_0;
+      if constexpr (!CLEAN) {
+        const unsigned w = mask_word<M_CELL_MAT>(m_n);
+        K = pick(w, Kp, K0);
+        G2 = pick(w, G2_p, G2_0);
+      }
       const CT exx = dxs(uxs_n - ux_n);
       const CT eyy = dys(uy_nn - uy_n);
       CT pp, txx, tyy;
@@ -621,45 +698,57 @@ struct MarchStage {
       } else {
         split_cell_trial(exx, eyy, K, G2, P0, pp, txx, tyy);
       }
-      const bool ok = (!EX || colC) && (!EY || (j + 1 >= 0 && j + 1 < nY));
-      if ((!CLEAN && (m_n & M_CELL_ZERO)) || !ok) {
-        pp = 0;
-        txx = 0;
-        tyy = 0;
+      if constexpr (!CLEAN) {
+        const unsigned w = mask_word<M_CELL_ZERO>(m_n);
+        pp = keep(w, pp);
+        txx = keep(w, txx);
+        tyy = keep(w, tyy);
       }
       tP_n = pp;
       tXX_n = txx;
       tYY_n = tyy;
     }
     const CT sXX_n = lane_next(tXX_n), sYY_n = lane_next(tYY_n);
+    const CT hXX_n = here(tXX_n + sXX_n), hYY_n = here(tYY_n + sYY_n);
+    const CT sxx = hXX_c + tXX_n + sXX_n, syy = hYY_c + tYY_n + sYY_n;  // vertex row j
     // trial vertex row j
     CT tXY_c;
     {
-      const CT g = CLEAN ? g0 : gt[(m_c >> M_VCLASS_SHIFT) & 15];
+      const CT g = CLEAN ? g0 : vert_mod(gt, m_c);
       CT txy;
       if constexpr (sizeof(CT) == 8) txy = g * (dys(uxs_n - uxs_c) + dxs(uys_n - uy_n));
       else txy = split_vertex_trial(g, (CT)(uxs_n - uxs_c), rdYc, (CT)(uys_n - uy_n), rdXc);
-      const bool ok = (!EX || colV) && (!EY || (j >= 0 && j < nY - 1));
-      if ((!CLEAN && (m_c & M_VERT_ZERO)) || !ok) txy = 0;
+      if constexpr (!CLEAN) txy = keep(mask_word<M_VERT_ZERO>(m_c), txy);
       tXY_c = txy;
     }
+    // the vertex row's values in the block of this lane's cell (columns 0 and
+    // nX-1: of the two columns next to the edge), and the block's sum
+    const CT pr_c = lane_prev(tXY_c);
+    CT f_c = pr_c, t_c = tXY_c;
+    if constexpr (EX) {
+      const CT nx = lane_next(tXY_c), pp = lane_prev(pr_c);
+      f_c = leftEdge ? tXY_c : rightEdge ? pp : pr_c;
+      t_c = leftEdge ? nx : rightEdge ? pr_c : tXY_c;
+    }
+    const CT hXY_c = here(f_c + t_c);
+    const CT n_c = hXY_p + f_c + t_c;
     // return mapping
     CT cXY_c = tXY_c, cP_c = tP_c, cXX_c = tXX_c, cYY_c = tYY_c;
-    if (plastic && !EDGE) {
-      // M::vertex_rm and M::cell_rm, with the scaling skipped where no lane
-      // of the wave yields (the squared invariants decide, as there)
-      const CT sxx = tXX_c + sXX_c + tXX_n + sXX_n;
-      const CT syy = tYY_c + sYY_c + tYY_n + sYY_n;
-      CT s2v, s2c;
-      if constexpr (sizeof(CT) == 8)
+    const bool pl = PL < 0 ? plastic : PL != 0;
+    if (pl) {
+      // the squared invariants decide; the scaling is skipped where no lane of
+      // the wave yields (stresses outside the grid do not count)
+      CT s2v, s2c, n = n_c;
+      if (EY && j == nY - 1) n = nXY_p;  // the two vertex rows above row nY-1
+      const CT av = (CT)0.25 * n;
+      if constexpr (sizeof(CT) == 8) {
         s2v = (CT)0.0625 * sxx * sxx + (CT)0.0625 * syy * syy + (CT)2.0 * tXY_c * tXY_c;
-      else
+        s2c = cXX_c * cXX_c + cYY_c * cYY_c + (CT)2.0 * av * av;
+      } else {
         s2v = split_s2_vertex(sxx, syy, tXY_c);
-      const CT pr_p = lane_prev(tXY_p), pr_c = lane_prev(tXY_c);
-      const CT av = (CT)0.25 * (pr_p + tXY_p + pr_c + tXY_c);
-      if constexpr (sizeof(CT) == 8) s2c = cXX_c * cXX_c + cYY_c * cYY_c + (CT)2.0 * av * av;
-      else s2c = split_s2_cell(cXX_c, cYY_c, av);
-      if (__any(s2v > c2lo || s2c > c2lo)) {
+        s2c = split_s2_cell(cXX_c, cYY_c, av);
+      }
+      if (__any((s2v > c2lo && (!EX || colV)) || (s2c > c2lo && (!EX || colC)))) {
         CT sc;
         if (rm_scale(s2v, coh, c2lo, sc)) cXY_c *= sc;
         if (rm_scale(s2c, coh, c2lo, sc)) {
@@ -667,51 +756,26 @@ struct MarchStage {
           cYY_c = cYY_c * sc;
         }
       }
-    } else if (plastic) {
-      const bool vok = (!EX || colV) && (!EY || (j >= 0 && j < nY - 1));
-      const CT sxx = tXX_c + sXX_c + tXX_n + sXX_n;
-      const CT syy = tYY_c + sYY_c + tYY_n + sYY_n;
-      if (vok) cXY_c = M::vertex_rm(tXY_c, sxx, syy, coh, c2lo);
-      const CT pr_p = lane_prev(tXY_p), pr_c = lane_prev(tXY_c);
-      {
-        // the clamped vertex blocks of the boundary columns (EX only): one
-        // column right and two left
-        CT nx_p = 0, nx_c = 0, nx_pp = 0, pp_p = 0, pp_c = 0, pp_pp = 0;
-        const CT pr_pp = lane_prev(tXY_pp);
-        if constexpr (EX) {
-          nx_p = lane_next(tXY_p);
-          nx_c = lane_next(tXY_c);
-          nx_pp = lane_next(tXY_pp);
-          pp_p = lane_prev(pr_p);
-          pp_c = lane_prev(pr_c);
-          pp_pp = lane_prev(pr_pp);
-        }
-        auto first = [&](CT t, CT pr, CT pp) { return leftEdge ? t : (rightEdge ? pp : pr); };
-        auto second = [&](CT t, CT pr, CT nxv) { return leftEdge ? nxv : (rightEdge ? pr : t); };
-        if (colC && (!EY || (j >= 1 && j < nY - 1))) {
-          const CT av = (CT)0.25 * (first(tXY_p, pr_p, pp_p) + second(tXY_p, pr_p, nx_p) +
-                                    first(tXY_c, pr_c, pp_c) + second(tXY_c, pr_c, nx_c));
-          M::cell_rm(cXX_c, cYY_c, av, coh, c2lo);
-        } else if (EY && colC && j == nY - 1 && j >= 1) {
-          const CT av = (CT)0.25 * (first(tXY_pp, pr_pp, pp_pp) + second(tXY_pp, pr_pp, nx_pp) +
-                                    first(tXY_p, pr_p, pp_p) + second(tXY_p, pr_p, nx_p));
-          M::cell_rm(cXX_c, cYY_c, av, coh, c2lo);
-        }
-        if (EY && j == 1) {
-          CT xx = tXX_p, yy = tYY_p;
-          if (colC) {
-            const CT av = (CT)0.25 * (first(tXY_p, pr_p, pp_p) + second(tXY_p, pr_p, nx_p) +
-                                      first(tXY_c, pr_c, pp_c) + second(tXY_c, pr_c, nx_c));
-            M::cell_rm(xx, yy, av, coh, c2lo);
-          }
-          cP_p = tP_p;
-          cYY_p = yy;
-        }
+      if (EY && j == 1) {
+        // cell row 0, from vertex rows 0 and 1 (its own step did not have them)
+        CT xx = tXX_p, yy = tYY_p;
+        M::cell_rm(xx, yy, (CT)0.25 * n_c, coh, c2lo);
+        cYY_p = yy;
       }
     }
     // velocity and displacement of row j
     const CT rP = lane_prev(cP_c), rXX = lane_prev(cXX_c);
-    const CT rXY_c = lane_prev(cXY_c), rXY_p = lane_prev(cXY_p);
+    // FP32 takes the left neighbours' difference as the shifted difference (the
+    // same value), the shift an operand of what follows; FP64, whose shifts
+    // are two moves each, carries them to the next step
+    CT dXY, rXY_c = 0;
+    if constexpr (sizeof(CT) == 8) {
+      rXY_c = lane_prev(cXY_c);
+      dXY = rXY_c - rXY_p;
+    } else {
+      dXY = lane_prev(cXY_c - cXY_p);
+      rXY_p = lane_prev(cXY_p);
+    }
     Out o;
     CT vx = vx_in, vy = vy_in;
     o.updX = (!EX || (i > 0 && i < nX)) && (!EY || (j > 0 && j < nY - 1));
@@ -720,27 +784,29 @@ struct MarchStage {
       // U advances with the velocity before its rounding to the storage type
       // (as the tile and march kernels do); the next stage gets the stored value
       if (o.updX)
-        vx = vx * vdampX + dTrho * (dxs(-cP_c + rP + cXX_c - rXX) + dys(rXY_c - rXY_p));
+        vx = vx * vdampX + dTrho * (dxs(-cP_c + rP + cXX_c - rXX) + dys(dXY));
       if (o.updY)
         vy = vy * vdampY + dTrho * (dys(-cP_c + cP_p + cYY_c - cYY_p) + dxs(cXY_p - rXY_p));
     } else {
       if (o.updX)
         vx = (CT)(VT)split_velocity(vx, vdampX, dTrho, -cP_c + rP + cXX_c - rXX, rdXc,
-                                    rXY_c - rXY_p, rdYc);
+                                    dXY, rdYc);
       if (o.updY)
         vy = (CT)(VT)split_velocity(vy, vdampY, dTrho, -cP_c + cP_p + cYY_c - cYY_p, rdYc,
                                     cXY_p - rXY_p, rdXc);
     }
-    const bool in = (!EX || inX) && (!EY || (j >= 0 && j < nY));
     o.vx = (CT)(VT)vx;
     o.vy = (CT)(VT)vy;
     if constexpr (sizeof(CT) == 8) {
-      o.ux = in ? ux_c + (double)vx * dT : ux_c;
-      o.uy = in ? uy_c + (double)vy * dT : uy_c;
+      o.ux = ux_c + (double)vx * dT;
+      o.uy = uy_c + (double)vy * dT;
     } else {
-      o.ux = in ? split_disp(ux_c, vx, dT) : ux_c;
-      o.uy = in ? split_disp(uy_c, vy, dT) : uy_c;
+      o.ux = split_disp(ux_c, vx, dT);
+      o.uy = split_disp(uy_c, vy, dT);
     }
+    // Ux column nX and Uy row nY are never updated
+    if ((EX && i >= nX) || (EY && j >= nY)) o.ux = ux_c;
+    if (EY && j >= nY) o.uy = uy_c;
     // rotate
     ux_c = ux_n;
     uxs_c = uxs_n;
@@ -753,16 +819,130 @@ struct MarchStage {
     tP_c = tP_n;
     tXX_c = tXX_n;
     tYY_c = tYY_n;
-    sXX_c = sXX_n;
-    sYY_c = sYY_n;
-    tXY_pp = tXY_p;
-    tXY_p = tXY_c;
+    hXX_c = hXX_n;
+    hYY_c = hYY_n;
+    hXY_p = hXY_c;
+    nXY_p = n_c;
     cP_p = cP_c;
     cYY_p = cYY_c;
     cXY_p = cXY_c;
+    rXY_p = rXY_c;
     return o;
   }
 };
+
+// Stage A's inputs in a two-iteration segment: the first rows (start) and,
+// for step t, Ux row t+1, Uy row t+2, mask row t+1 and V row t of the state in
+// HBM, through buffer resources (the lane's byte offset fixed, the row's in an
+// SGPR).  Interior segments clamp rows to the segment's last step tEnd.  Edge
+// segments bound each resource to its field: lanes outside the field's
+// columns carry the offset kOob, and a row outside the field reads through a
+// resource of bound 0, so every such load returns 0 without a branch.
+template <typename CT, typename VT, bool EX, bool EY = EX, bool CLEAN = false>
+struct StageInput {
+  static constexpr bool EDGE = EX || EY;
+  using Ld = typename March<CT, VT>::Ld;
+  const double* Uxi;
+  const double* Uyi;
+  const VT* Vxi;
+  const VT* Vyi;
+  const unsigned char* mask;
+  int nX, nY, sx, i, tEnd;
+  unsigned o8, oV;
+  __amdgpu_buffer_rsrc_t bUx, bUy, bVx, bVy, bM;
+  // edge segments: lane offsets with the column test folded in (Ux columns
+  // 0..nX, the others 0..nX-1; V is read for columns 0..nX-1 only)
+  unsigned oUx, oC8, oM, oVc;
+
+  __device__ __forceinline__ StageInput(const RveDev& r, int cur, int vpar, int col, int tEnd_)
+      : Uxi(r.Ux[cur]), Uyi(r.Uy[cur]),
+        Vxi(static_cast<const VT*>(vpar ? r.Vx2 : r.Vx)),
+        Vyi(static_cast<const VT*>(vpar ? r.Vy2 : r.Vy)), mask(r.mask), nX(r.nX), nY(r.nY),
+        sx(r.nX + 1), i(col), tEnd(tEnd_), o8((unsigned)col * 8u),
+        oV((unsigned)col * (unsigned)sizeof(VT)) {
+    if (!EDGE) {
+      bUx = brsrc(Uxi);
+      bUy = brsrc(Uyi);
+      bVx = brsrc(Vxi);
+      bVy = brsrc(Vyi);
+      bM = brsrc(mask);
+    } else {
+      const unsigned ux = (unsigned)nY * (unsigned)sx, uy = (unsigned)(nY + 1) * (unsigned)nX;
+      bUx = brsrc_n(Uxi, ux * 8u);
+      bUy = brsrc_n(Uyi, uy * 8u);
+      bVx = brsrc_n(Vxi, ux * (unsigned)sizeof(VT));
+      bVy = brsrc_n(Vyi, uy * (unsigned)sizeof(VT));
+      bM = brsrc_n(mask, (unsigned)nY * (unsigned)nX);
+      const bool cx = col >= 0 && col <= nX, cc = col >= 0 && col < nX;
+      oUx = cx ? o8 : kOob;
+      oC8 = cc ? o8 : kOob;
+      oM = cc ? (unsigned)col : kOob;
+      oVc = cc ? oV : kOob;
+    }
+  }
+
+  // Ux row jb, Uy row jb+1, mask row jb into the stage
+  template <int PL>
+  __device__ __forceinline__ void start(MarchStage<CT, VT, EX, EY, CLEAN, PL>& st, int jb) const {
+    double ux = 0.0, uy = 0.0;
+    unsigned m = 0;
+    const bool colC = !EDGE || (i >= 0 && i < nX);
+    if (!EDGE) {
+      ux = gld(Uxi, (unsigned)(jb * sx + i));
+      uy = gld(Uyi, (unsigned)((jb + 1) * nX + i));
+      if (!CLEAN) m = gld(mask, (unsigned)(jb * nX + i));
+    } else {
+      if (i >= 0 && i <= nX && jb >= 0 && jb < nY) ux = gld(Uxi, (unsigned)(jb * sx + i));
+      if (colC && jb + 1 >= 0 && jb + 1 <= nY) uy = gld(Uyi, (unsigned)((jb + 1) * nX + i));
+      if (!CLEAN && colC && jb >= 0 && jb < nY) m = gld(mask, (unsigned)(jb * nX + i));
+    }
+    st.start(ux, uy, stage_mask(m));
+  }
+
+  __device__ __forceinline__ Ld fetch(int t0) const {
+    const int t = EDGE ? t0 : min(t0, tEnd);
+    Ld d;
+    if (!EDGE) {
+      d.ux = bld<double>(bUx, o8, (unsigned)(t + 1) * (unsigned)sx * 8u);
+      d.uy = bld<double>(bUy, o8, (unsigned)(t + 2) * (unsigned)nX * 8u);
+      d.m = CLEAN ? 0u : bld<unsigned char>(bM, (unsigned)i, (unsigned)(t + 1) * (unsigned)nX);
+      d.vx = bld<VT>(bVx, oV, (unsigned)t * (unsigned)sx * (unsigned)sizeof(VT));
+      d.vy = bld<VT>(bVy, oV, (unsigned)t * (unsigned)nX * (unsigned)sizeof(VT));
+    } else {
+      // rows outside a field read through a resource of bound 0 (the row
+      // tests are uniform: scalar selects); the row offset is then 0
+      const __amdgpu_buffer_rsrc_t none = brsrc_n(Uxi, 0u);
+      const bool r1 = t + 1 >= 0 && t + 1 < nY, r2 = t + 2 >= 0 && t + 2 <= nY,
+                 r0 = t >= 0 && t < nY;
+      const unsigned s1 = r1 ? (unsigned)(t + 1) : 0u, s2 = r2 ? (unsigned)(t + 2) : 0u,
+                     s0 = r0 ? (unsigned)t : 0u;
+      d.ux = bld<double>(r1 ? bUx : none, oUx, s1 * (unsigned)sx * 8u);
+      d.uy = bld<double>(r2 ? bUy : none, oC8, s2 * (unsigned)nX * 8u);
+      d.m = CLEAN ? 0u : bld<unsigned char>(r1 ? bM : none, oM, s1 * (unsigned)nX);
+      d.vx = bld<VT>(r0 ? bVx : none, oVc, s0 * (unsigned)sx * (unsigned)sizeof(VT));
+      d.vy = bld<VT>(r0 ? bVy : none, oVc, s0 * (unsigned)nX * (unsigned)sizeof(VT));
+    }
+    return d;
+  }
+};
+
+// Whether the mask is 0 over rows [jlo, jhi] and columns [ilo, ihi] (clipped
+// to the grid), from the block map; the same answer in every lane.
+__device__ __forceinline__ bool mask_clear(const RveDev& r, int ilo, int ihi, int jlo, int jhi) {
+  ilo = max(ilo, 0);
+  jlo = max(jlo, 0);
+  ihi = min(ihi, r.nX - 1);
+  jhi = min(jhi, r.nY - 1);
+  if (ilo > ihi || jlo > jhi) return true;
+  const int bx0 = ilo / kMapCols, bx1 = ihi / kMapCols;
+  const int by0 = jlo / kMapRows, by1 = jhi / kMapRows;
+  const int nbx = (r.nX + kMapCols - 1) / kMapCols;
+  const int w = bx1 - bx0 + 1, n = w * (by1 - by0 + 1);
+  unsigned any = 0;
+  for (int q = (int)(threadIdx.x & 63); q < n; q += 64)
+    any |= r.mmap[(by0 + q / w) * nbx + bx0 + q % w];
+  return !__any(any != 0);
+}
 
 }  // namespace
 
