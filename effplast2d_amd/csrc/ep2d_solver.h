@@ -204,6 +204,14 @@ class Solver {
   bool settled();                   // after the stream is synchronised
   void settle();
   void iterateLaunches(long n);
+  // a run of plain iterations as a graph (replayPlain), and the RVE record its
+  // launches were captured with
+  hipGraph_t plainGraph_ = nullptr;
+  hipGraphExec_t plainExec_ = nullptr;
+  RveDev plainRve_;
+  long plainIters_ = 0;             // iterations asked for so far
+  long replayPlain(long n);
+  void dropPlainGraph();
   std::pair<hipEvent_t, hipEvent_t> takeTimingEvents();
   void launchMulti(int q);         // ipl_ iterations, q-th such launch of a run
   void launchClose(int ns, int q);  // ns = 3 or 2 iterations closing a run
