@@ -226,7 +226,7 @@ struct ResRows {
   static constexpr bool F64 = sizeof(CT) == 8;
   const CT* gt;
   int nX, nY, i;
-  bool colC, leftEdge, rightEdge, plastic;
+  bool colC, leftEdge, rightEdge, plastic, near;
   CT coh, c2lo, K0, Kp, G2_0, G2_p, P0, vdampX, vdampY, dTrho, g0;
   double dT, dXd, dYd, rdXd, rdYd;
   CT rdXc, rdYc;
@@ -265,6 +265,7 @@ struct ResRows {
     leftEdge = EX && i == 0;
     rightEdge = EX && i == nX - 1;
     plastic = r.plastic != 0;
+    near = rm_near(r.coh);
     coh = uni(r.coh);
     if constexpr (F64) c2lo = r.coh2lo;
     else c2lo = r.coh2lof;
@@ -392,12 +393,7 @@ struct ResRows {
     };
     auto scale = [&](auto KK) {
       constexpr int k = decltype(KK)::value;
-      CT sc;
-      if (rm_scale(s2v[k + 1], coh, c2lo, sc)) cXY[k + 1] *= sc;
-      if (rm_scale(s2c[k + 1], coh, c2lo, sc)) {
-        cXX[k + 1] = cXX[k + 1] * sc;
-        cYY[k + 1] = cYY[k + 1] * sc;
-      }
+      rm_both<true>(s2v[k + 1], s2c[k + 1], coh, c2lo, near, cXY[k + 1], cXX[k + 1], cYY[k + 1]);
     };
     auto move = [&](auto KK) {  // velocity and displacement of row k
       constexpr int k = decltype(KK)::value;
