@@ -9,11 +9,11 @@
 // which is why a tile computes T = 2 iterations between exchanges, on a halo
 // of 2T nodes that it takes over from its neighbours.
 //
-// us per iteration, single RVE (tile kernel, one iteration a launch; chain
-// kernels; here):
+// us per iteration, single RVE (tile kernel, one iteration a launch, before there
+// were resident runs; chain kernels; here):
 //            64^2             256^2            333^2            512^2
-//   FP64     7.5 / 5.8 / 4.4  6.8 / 6.6 / 4.4  7.1 / 7.0 / 4.5  8.9 / 8.2 / 6.9
-//   split    6.6 / 3.5 / 2.6  6.0 / 3.6 / 2.7  6.3 / 4.3 / 3.1  7.2 / 4.6 / 4.0
+//   FP64     7.5 / 4.7 / 4.1  6.8 / 5.4 / 4.0  7.3 / 5.8 / 4.2  8.9 / 6.9 / 6.2
+//   split    6.8 / 3.1 / 2.6  6.0 / 3.3 / 2.6  6.5 / 3.9 / 3.0  7.2 / 4.3 / 3.9
 // T = 1 took 4.3 (FP64) and 3.1 (split) on the small grids.
 //
 // Layout.  Lane L of every wave is column s+L of the tile's region, wave v
@@ -200,7 +200,7 @@ struct ResLds {
   VT rowV[T > 1 ? 4 * T : 1][2][64];
   double2 zeroU[R][4 * T];
   VT zeroV[T > 1 ? R : 1][4 * T][2];
-  CT gt[16];
+  VertMod<CT> gt[16];
   unsigned state;
 };
 
@@ -224,7 +224,7 @@ template <typename CT, typename VT, int R, int C, bool EX, bool EY, bool CLEAN>
 struct ResRows {
   using M = March<CT, VT>;
   static constexpr bool F64 = sizeof(CT) == 8;
-  const CT* gt;
+  const VertMod<CT>* gt;
   int nX, nY, i;
   bool colC, leftEdge, rightEdge, plastic, near;
   CT coh, c2lo, K0, Kp, G2_0, G2_p, P0, vdampX, vdampY, dTrho, g0;
@@ -256,7 +256,7 @@ struct ResRows {
       return __builtin_bit_cast(
           float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, (float)a)));
   }
-  __device__ __forceinline__ void setup(const RveDev& r, const CT* g, int col) {
+  __device__ __forceinline__ void setup(const RveDev& r, const VertMod<CT>* g, int col) {
     gt = g;
     nX = r.nX;
     nY = r.nY;
@@ -296,14 +296,16 @@ struct ResRows {
   }
 
   // rows -2 .. R of Ux and of the vertices at index k + 2, rows -1 .. R+1 of Uy
-  // and rows -1 .. R of the cells at index k + 1; mask(k): the mask byte of row
+  // and rows -1 .. R of the cells at index k + 1; mask: the mask bytes of rows
   // k - 2
   template <typename Mask>
   __device__ __forceinline__ void iterate(int jw, double (&ux)[R], double (&uy)[R], VT (&vx)[R],
                                           VT (&vy)[R], double a0, double a1, double b1,
-                                          double c0, double d0, double d1, Mask mask) const {
+                                          double c0, double d0, double d1, const Mask& mask) const {
     double sx[R + 3];  // Ux of the next column
-    CT tP[R + 2], tXX[R + 2], tYY[R + 2], sXX[R + 2], sYY[R + 2], tXY[R + 2];
+    CT tP[R + 2], tXX[R + 2], tYY[R + 2], tXY[R + 2];
+    CT vXX[R + 1], vYY[R + 1], nXY[R + 1];  // sums of vertex row and cell row k at k + 1
+    CT hXX = 0, hYY = 0, hXY = 0;
     CT cXX[R + 1], cYY[R + 1], cXY[R + 1];  // corrected rows -1 .. R-1 at k + 1
     // the rows before this iteration's updates reach them (row k is updated
     // after every use of its old value)
@@ -322,9 +324,12 @@ struct ResRows {
 
     auto cell = [&](auto KK) {  // trial cell of row k
       constexpr int k = decltype(KK)::value;
-      const unsigned mb = CLEAN ? 0u : mask(k + 2);
-      const CT K = !CLEAN && (mb & M_CELL_MAT) ? Kp : K0;
-      const CT G2 = !CLEAN && (mb & M_CELL_MAT) ? G2_p : G2_0;
+      CT K = K0, G2 = G2_0;
+      if constexpr (!CLEAN) {
+        const unsigned w = mask.template word<M_CELL_MAT, k + 2>();
+        K = pick(w, Kp, K0);
+        G2 = pick(w, G2_p, G2_0);
+      }
       const CT exx = dxs(sx[k + 2] - ox[k + 2]);
       const CT eyy = dys(oy[k + 2] - oy[k + 1]);
       CT pp, txx, tyy;
@@ -335,54 +340,68 @@ struct ResRows {
       } else {
         split_cell_trial(exx, eyy, K, G2, P0, pp, txx, tyy);
       }
-      if (!CLEAN && (mb & M_CELL_ZERO)) pp = 0, txx = 0, tyy = 0;
+      if constexpr (!CLEAN) {
+        const unsigned w = mask.template word<M_CELL_ZERO, k + 2>();
+        pp = keep(w, pp);
+        txx = keep(w, txx);
+        tyy = keep(w, tyy);
+      }
       tP[k + 1] = pp;
       tXX[k + 1] = txx;
       tYY[k + 1] = tyy;
-      sXX[k + 1] = lane_next(txx);
-      sYY[k + 1] = lane_next(tyy);
+      // the vertex row above's sums, and the start of this row's
+      const CT x = lane_next(txx), y = lane_next(tyy);
+      if constexpr (k >= 0) {
+        vXX[k] = hXX + txx + x;
+        vYY[k] = hYY + tyy + y;
+      }
+      hXX = txx + x;
+      hYY = tyy + y;
     };
     auto vertex = [&](auto KK) {  // trial vertex of row k
       constexpr int k = decltype(KK)::value;
-      const unsigned mb = CLEAN ? 0u : mask(k + 2);
-      const CT g = CLEAN ? g0 : gt[(mb >> M_VCLASS_SHIFT) & 15];
+      const CT g = CLEAN ? g0 : vert_mod(gt, CLEAN ? 0u : mask.byte(k + 2));
       const double uyn = oy[k + 2], uys = lane_next(uyn);
       CT t;
       if constexpr (F64) t = g * (dys(sx[k + 3] - sx[k + 2]) + dxs(uys - uyn));
       else t = split_vertex_trial(g, (CT)(sx[k + 3] - sx[k + 2]), rdYc, (CT)(uys - uyn), rdXc);
-      if (!CLEAN && (mb & M_VERT_ZERO)) t = 0;
+      if constexpr (!CLEAN) t = keep(mask.template word<M_VERT_ZERO, k + 2>(), t);
       tXY[k + 2] = t;
+    };
+    // the vertex row in the blocks of this lane's cell, clamped to the grid in x
+    // (EffPlast2D.cu:109-137), and the sum of the block of rows k-1 and k
+    // (lane 0 of the first strip is column 0: it keeps its own value)
+    auto block = [&](auto KK) {
+      constexpr int k = decltype(KK)::value;
+      const CT t = tXY[k + 2];
+      CT f = lane_prev_or(t), c = t;
+      if constexpr (EX) {
+        const CT nx = lane_next(t), pp = lane_prev(f);
+        c = leftEdge ? nx : rightEdge ? f : t;
+        f = rightEdge ? pp : f;
+      }
+      if constexpr (k > -2) nXY[k + 1] = hXY + f + c;
+      hXY = f + c;
     };
     // squared invariants of vertex and cell row k, and whether they may yield
     CT s2v[R + 1], s2c[R + 1];
     auto invariants = [&](auto KK) {
       constexpr int k = decltype(KK)::value;
       const int j = jw + k;
-      const CT sxx = tXX[k + 1] + sXX[k + 1] + tXX[k + 2] + sXX[k + 2];
-      const CT syy = tYY[k + 1] + sYY[k + 1] + tYY[k + 2] + sYY[k + 2];
+      const CT sxx = vXX[k + 1], syy = vYY[k + 1];
       const CT t = tXY[k + 2];
       if constexpr (F64)
         s2v[k + 1] = (CT)0.0625 * sxx * sxx + (CT)0.0625 * syy * syy + (CT)2.0 * t * t;
       else s2v[k + 1] = split_s2_vertex(sxx, syy, t);
-      // the 2x2 vertex block of the cell, clamped to the grid (EffPlast2D.cu:109-137)
-      CT p = tXY[k + 1], c = t;
+      CT n = nXY[k + 1];
       if constexpr (EY) {
-        // row 0, the first of its wave, takes rows 0 and 1, row nY-1 the two
-        // above it
-        if (k == 0 && j == 0) p = t, c = tXY[3];
-        else if (k >= 0 && j == nY - 1) p = tXY[k >= 0 ? k : 0], c = tXY[k + 1];
+        // row 0, the first of its wave, takes vertex rows 0 and 1, row nY-1 the
+        // two above it
+        const CT below = nXY[k == 0 ? 2 : k + 1], above = nXY[k >= 0 ? k : 0];
+        n = k >= 0 && j == nY - 1 ? above : n;
+        n = k == 0 && j == 0 ? below : n;
       }
-      // (lane 0 of the first strip is column 0: it keeps its own value)
-      CT f_p = lane_prev_or(p), f_c = lane_prev_or(c), s_p = p, s_c = c;
-      if constexpr (EX) {
-        const CT nx_p = lane_next(p), nx_c = lane_next(c), pp_p = lane_prev(f_p),
-                 pp_c = lane_prev(f_c);
-        s_p = leftEdge ? nx_p : rightEdge ? f_p : p;
-        s_c = leftEdge ? nx_c : rightEdge ? f_c : c;
-        f_p = rightEdge ? pp_p : f_p;
-        f_c = rightEdge ? pp_c : f_c;
-      }
-      const CT av = (CT)0.25 * (f_p + s_p + f_c + s_c);
+      const CT av = (CT)0.25 * n;
       const CT xx = tXX[k + 1], yy = tYY[k + 1];
       if constexpr (F64) s2c[k + 1] = xx * xx + yy * yy + (CT)2.0 * av * av;
       else s2c[k + 1] = split_s2_cell(xx, yy, av);
@@ -395,23 +414,34 @@ struct ResRows {
       constexpr int k = decltype(KK)::value;
       rm_both<true>(s2v[k + 1], s2c[k + 1], coh, c2lo, near, cXY[k + 1], cXX[k + 1], cYY[k + 1]);
     };
+    CT rXY = 0;
     auto move = [&](auto KK) {  // velocity and displacement of row k
       constexpr int k = decltype(KK)::value;
       const int j = jw + k;
       const CT cP = tP[k + 1], pP = tP[k], xx = cXX[k + 1], yy = cYY[k + 1], pY = cYY[k];
       const CT xyc = cXY[k + 1], xyp = cXY[k];
       const CT rP = lane_prev(cP), rXX = lane_prev(xx);
-      const CT rXYc = lane_prev(xyc), rXYp = lane_prev(xyp);
+      // the left neighbours' shear: FP32 shifts the difference (the same value)
+      CT dXY, rXYp;
+      if constexpr (F64) {
+        if constexpr (k == 0) rXY = lane_prev(xyp);
+        rXYp = rXY;
+        rXY = lane_prev(xyc);
+        dXY = rXY - rXYp;
+      } else {
+        rXYp = lane_prev(xyp);
+        dXY = lane_prev(xyc - xyp);
+      }
       CT wx = (CT)vx[k], wy = (CT)vy[k];
       // (V past the last column is nobody's)
       const bool updX = (!EX || !leftEdge) && (!EY || (j > 0 && j < nY - 1));
       const bool updY = (!EX || !(leftEdge || rightEdge)) && (!EY || (j > 0 && j < nY));
       if constexpr (F64) {
-        if (updX) wx = wx * vdampX + dTrho * (dxs(-cP + rP + xx - rXX) + dys(rXYc - rXYp));
+        if (updX) wx = wx * vdampX + dTrho * (dxs(-cP + rP + xx - rXX) + dys(dXY));
         if (updY) wy = wy * vdampY + dTrho * (dys(-cP + pP + yy - pY) + dxs(xyp - rXYp));
       } else {
         if (updX)
-          wx = (CT)(VT)split_velocity(wx, vdampX, dTrho, -cP + rP + xx - rXX, rdXc, rXYc - rXYp,
+          wx = (CT)(VT)split_velocity(wx, vdampX, dTrho, -cP + rP + xx - rXX, rdXc, dXY,
                                       rdYc);
         if (updY)
           wy = (CT)(VT)split_velocity(wy, vdampY, dTrho, -cP + pP + yy - pY, rdYc, xyp - rXYp,
@@ -439,7 +469,9 @@ struct ResRows {
       if constexpr (k0 == 0) {
         sx[2] = lane_next(ox[2]);
         vertex(N2{});
+        block(N2{});
         vertex(N1{});
+        block(N1{});
         cell(N1{});
         cell(std::integral_constant<int, 0>{});
       }
@@ -448,6 +480,7 @@ struct ResRows {
         sx[k + 3] = lane_next(ox[k + 3]);
         cell(std::integral_constant<int, k + 1>{});
         vertex(K);
+        block(K);
       });
       constexpr int f = k0 == 0 ? -1 : k0, fn = cn + (k0 == 0 ? 1 : 0);
       each<f, fn>([&](auto K) {
@@ -499,8 +532,10 @@ struct ResWave {
   VT vx[R], vy[R];
   unsigned mk[NM];  // mask bytes of rows jw-2 .. jw+R, four to a word
 
-  __device__ __forceinline__ unsigned m(int k) const {
-    return CLEAN ? 0u : (mk[k >> 2] >> (8 * (k & 3))) & 0xffu;
+  __device__ __forceinline__ unsigned byte(int k) const { return mk[k >> 2] >> (8 * (k & 3)); }
+  template <int BIT, int k>
+  __device__ __forceinline__ unsigned word() const {
+    return mask_word<BIT << (8 * (k & 3))>(mk[k >> 2]);
   }
 
   __device__ __forceinline__ void run(const RveDev& r, const ResTile& q, int cur, VT* Vx, VT* Vy,
@@ -538,6 +573,8 @@ struct ResWave {
           if (inCol && j >= 0 && j < nY)
             mk[k >> 2] |= (unsigned)gld(r.mask, (unsigned)(j * nX + i)) << (8 * (k & 3));
         }
+#pragma unroll
+        for (int k = 0; k < NM; k++) mk[k] ^= 0x01010101u * (unsigned)(M_CELL_ZERO | M_VERT_ZERO);
       }
     }
 
@@ -737,7 +774,7 @@ struct ResWave {
       // U of the state before the last iteration: the stress fields of a load
       // step are recomputed from it (EffPlast2D.cu:428)
       if (t == n - 1) storeU(r, q, cur, i, jw, own);
-      st.iterate(jw, ux, uy, vx, vy, a0, a1, b1, c0, d0, d1, [&](int k) { return m(k); });
+      st.iterate(jw, ux, uy, vx, vy, a0, a1, b1, c0, d0, d1, *this);
     }
     storeU(r, q, cur ^ 1, i, jw, own);
 #pragma unroll
@@ -765,15 +802,15 @@ struct ResWave {
   }
 };
 
-// waves of a SIMD the registers are held to: two tiles to a CU in the split
-// scheme, one in FP64
-template <typename CT>
+// waves of a SIMD the registers are held to: two tiles to a CU where they are
+// given half of one (two split rows a wave), else one
+template <typename CT, int R>
 constexpr int res_waves() {
-  return sizeof(CT) == 4 ? 4 : 2;
+  return sizeof(CT) == 4 && R <= 2 ? 4 : 2;
 }
 
 template <typename CT, typename VT, int R, int T, int NW>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(res_waves<CT>()))) void k_resident(
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(res_waves<CT, R>()))) void k_resident(
     const RveDev* __restrict__ rves, const ResTile* __restrict__ tiles, int parity, int vpar,
     int n, const char* xch, unsigned xpar, unsigned tag0, ResCtl* ctl, unsigned cost,
     unsigned cap, unsigned* told) {
@@ -782,7 +819,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(res_wav
   const int v = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const ResTile q = tiles[blockIdx.x];
   const RveDev& r = rves[q.rve];
-  if (threadIdx.x < 16) lds.gt[threadIdx.x] = (CT)r.gtab[threadIdx.x];
+  if (threadIdx.x < 16) lds.gt[threadIdx.x].g = (CT)r.gtab[threadIdx.x];
   if (threadIdx.x < R * 4 * T) {
     (&lds.zeroU[0][0])[threadIdx.x] = make_double2(0.0, 0.0);
     if constexpr (T > 1) {
@@ -860,19 +897,21 @@ int res_parts(int n, int span, int T) {
 
 }  // namespace
 
-// From runs of 500 iterations of one RVE (us per iteration; the chains beside
-// them on the shortest segments of one round):
-//   split, waves of two rows:  64^2 2.6 (chains 3.5), 256^2 2.7 (3.6), 333^2
-//     3.1 (4.3), with two tiles to a CU 352^2 3.4 (4.3); 400^2 4.1, as four rows
-//   split, four rows, one tile to a CU:  450^2 4.3 (4.7), 560^2 4.0 (4.8); with
-//     two tiles to a CU 640^2 5.3 (5.0): the chains there and beyond
-//   FP64, two rows:  64^2 4.4 (5.8), 256^2 4.4 (6.6), 333^2 4.5 (7.0)
-//   FP64, four rows:  352^2 6.8 (7.0), 560^2 6.9 (8.7)
-//   FP64, six rows, an exchange each iteration:  600^2 9.5 (9.1), 640^2 9.5
-//     (9.2), 700^2 9.2 (10.1), 768^2 9.3 (11.0); beyond, the tiles find no room
+// From runs of 500 iterations of one RVE whose nodes yield (us per iteration; in
+// brackets the chains on the shortest segments of one round):
+//   split, two rows a wave:  64^2 2.6 (3.1), 256^2 2.6 (3.3), 333^2 3.0 (3.9),
+//     with two tiles to a CU 352^2 3.4 (3.9)
+//   split, four rows, one tile to a CU:  400^2 4.1 (4.0), 450^2 4.2 (4.3), 512^2
+//     3.9 (4.3), 560^2 4.1 (4.5); with two tiles to a CU the chains were faster
+//   FP64, two rows:  64^2 4.1 (4.7), 256^2 4.0 (5.4), 333^2 4.2 (5.8)
+//   FP64, four rows:  352^2 6.2 (5.9), 400^2 6.3 (6.3), 450^2 6.4 (6.5), 512^2
+//     6.2 (6.9), 560^2 6.2 (7.2)
+//   FP64, six rows, an exchange each iteration:  672^2 8.2 (8.3), 700^2 8.0 (8.4),
+//     768^2 8.3 (9.2); beyond, the tiles find no room.  600^2 and 640^2 lie past
+//     the four rows' room: chains, 7.5
 std::vector<ResShape> resident_shapes(int mode) {
-  if (mode == 2) return {{2, 2, 8, 1, 0}, {4, 2, 8, 2, 0}};
-  return {{2, 2, 8, 2, 0}, {4, 2, 8, 2, 0}, {6, 1, 8, 2, 672}};
+  if (mode == 2) return {{2, 2, 8, 1, 0}, {4, 2, 8, 2, 448}};
+  return {{2, 2, 8, 2, 0}, {4, 2, 8, 2, 448}, {6, 1, 8, 2, 672}};
 }
 
 int resident_tiles(const ResShape& sh, int mode, int n, int rve, size_t x0, ResTile* out,
