@@ -1480,13 +1480,16 @@ __device__ __forceinline__ void chain_run(const RveDev& r, int cur, int vpar, in
 //
 // One segment per workgroup of NS x W waves (stage k on waves kW .. kW+W-1,
 // wave c of a stage on columns s+60c ..).  The split scheme's register
-// budget holds seven waves per SIMD (six with two waves per stage, where the
-// LDS of three workgroups of eight waves fills a CU); FP64 chains of one
+// budget holds six waves per SIMD (with two waves per stage the LDS of three
+// workgroups of eight waves fills a CU; with one, seven waves spilled 14
+// registers: 20 x 1024^2, one wave, 128 rows, took 82.0 us an iteration over a
+// plastic run against 82.4, but 70.9 against 73.5 in the tuning launches on the
+// fresh state, so the batch chose it over two waves' 77.9).  FP64 chains of one
 // wave per stage are held to five (a few registers spilled, 2-4% faster than
 // four), with two waves per stage they run four.
 template <typename CT, typename VT, int NS, int W>
 __global__ __launch_bounds__(64 * NS * W)
-__attribute__((amdgpu_waves_per_eu(sizeof(CT) == 4 ? (W == 1 ? 7 : 6) : (W == 1 ? 5 : 1)))) void k_chain(const RveDev* __restrict__ rves,
+__attribute__((amdgpu_waves_per_eu(sizeof(CT) == 4 ? 6 : (W == 1 ? 5 : 1)))) void k_chain(const RveDev* __restrict__ rves,
                                                    const int4* __restrict__ segs, int nsegs,
                                                    int parity, int vpar) {
   constexpr int UW = 60 * W + 4;
