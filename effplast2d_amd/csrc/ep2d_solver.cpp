@@ -285,11 +285,13 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
     // chains with two waves per stage (four iterations per launch, in the
     // launch order of chain_work_order).  Up to 1024^2 the shortest segments
     // whose workgroups the device holds in one round (14 rows for split, 21
-    // for FP64 on 256 CUs at 1024^2: 7.1 and 14.7 us per iteration; 16 split
-    // rows take 8.6, 20 FP64 rows 17.3 and the FP64 tile kernel 16.7; at
-    // 1000^2 7.1 and 14.7 against 13.2 and 18.4 on the tile kernel, at 256^2
-    // 3.6 and 6.0 against 6.0 and 6.8), 48 rows at 2048^2 and 96 beyond
-    // (split 16.4 and 57.6 us, FP64 43.0 and 124.3 against 47.6 and 154.7 on
+    // for FP64 on 256 CUs at 1024^2: 6.5 and 12.0 us per iteration; 16 split
+    // rows take 6.8, 20 FP64 rows 13.3 and the FP64 tile kernel 16.3; at
+    // 1000^2 6.7 and 11.6 against 13.2 and 18.4 on the tile kernel, at 256^2
+    // 3.3 and 5.4 against 6.0 and 6.8), 48 rows at 2048^2 and 96 beyond
+    // (split 14.3 and 54 us, FP64 34 and 104; before the boundary strips ran
+    // the interior's expressions 16.4 and 57.6, 43.0 and 124.3, and 47.6 and
+    // 154.7 in FP64 on
     // wave pairs).  Runs of kResMinIters iterations and more of a grid that
     // fits on the chip take the resident kernel (planResident) instead.
     const int n = std::max(nX, nY);
