@@ -1466,7 +1466,8 @@ __device__ __forceinline__ void chain_run(const RveDev& r, int cur, int vpar, in
 // them, those at the left and right boundary.  Steps that got it here, us per
 // iteration before and after: 1024^2 split 7.2 -> 6.4, FP64 14.7 -> 13.7;
 // 2048^2 split 15.2 -> 14.1, FP64 41.4 -> 36.0; 4096^2 split 55.4 -> 54.0 (the
-// HBM traffic of 52 bytes a node and launch is 4 TB/s there), FP64 121.5 -> 115.0.
+// HBM traffic of 52 bytes a node and launch is 4 TB/s there), FP64 121.5 -> 115.0
+// (with rm_both 12.0, 34 and 104 where every node yields).
 // - Plastic and elastic interior segments have code of their own, and no lane
 //   branch: a step is one block of code up to the scaling.
 // - Carried sums (MarchStage) make a lane shift an operand of an addition.
