@@ -371,6 +371,10 @@ int ep2d_diag_chain_order(const int* segs, int n, int stageWaves, const int* dim
   });
 }
 
+int ep2d_diag_resident(ep2d_handle* h, const long long* limits, long long* counts) {
+  return guarded([&] { S(h)->diagResident(limits, counts); });
+}
+
 int ep2d_diag_copy(int device, size_t bytes, int reps, double* avgMs) {
   return guarded([&] {
     if (!avgMs || reps < 1 || bytes < 16 || bytes > ((size_t)64 << 30))

@@ -201,6 +201,12 @@ struct ResTile {
 struct ResCtl {
   unsigned arrive, state, depart, pad;
 };
+// Bounds of a launch's waits: for its other tiles (ticks of 10 ns; 0: it is
+// turned away at once) and for the words of one exchange (polls of about a
+// microsecond).
+struct ResLimits {
+  unsigned arriveTicks = 25000000u, polls = 1u << 20;
+};
 // how a launch went: run, or ended with the fields untouched because other
 // launches hold the GPU's room or its tiles did not all start in time; lost:
 // a wait inside the run ended at its bound (the fields are not valid)
@@ -220,6 +226,7 @@ struct ResLaunch {
   unsigned tag0;            // tags tag0 + 1 .. tag0 + iters, none used before
   ResCtl* ctl;
   unsigned cost, room;      // half CUs of a tile, and of the device
+  ResLimits limits;
   unsigned* told;           // pinned host word that receives how the launch went
 };
 // The shapes of a scheme, from the smallest tiles to the largest: a grid takes

@@ -53,11 +53,6 @@ namespace {
 // tiles in flight on this device, in half CUs
 __device__ unsigned g_resInUse;
 
-// waits for the launch's other tiles (100 MHz ticks), and for one exchange
-// (polls of about a microsecond)
-constexpr unsigned long long kArriveTicks = 25000000ull;
-constexpr unsigned kPollLimit = 1u << 20;
-
 __device__ __forceinline__ unsigned ald(unsigned* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -74,14 +69,15 @@ __device__ __forceinline__ unsigned acas(unsigned* p, unsigned from, unsigned to
 // first to arrive decides: it reserves the room, waits for the others and
 // lets the run go, or ends it.  (The others' bound is longer: it only serves
 // if the first never decides.)
-__device__ unsigned res_arrive(ResCtl* c, unsigned tiles, unsigned cost, unsigned cap) {
+__device__ unsigned res_arrive(ResCtl* c, unsigned tiles, unsigned cost, unsigned cap,
+                               unsigned ticks) {
   const unsigned long long t0 = wall_clock64();
   if (aadd(&c->arrive, 1u) == 0) {
     const unsigned need = tiles * cost;
-    unsigned how = kResGo;
+    unsigned how = ticks ? kResGo : kResLate;
     if (aadd(&g_resInUse, need) + need > cap) how = kResNoRoom;
     while (how == kResGo && ald(&c->arrive) < tiles) {
-      if (wall_clock64() - t0 > kArriveTicks) how = kResLate;
+      if (wall_clock64() - t0 > ticks) how = kResLate;
       __builtin_amdgcn_s_sleep(1);
     }
     const unsigned was = acas(&c->state, 0u, how);
@@ -90,7 +86,7 @@ __device__ unsigned res_arrive(ResCtl* c, unsigned tiles, unsigned cost, unsigne
   for (;;) {
     const unsigned s = ald(&c->state);
     if (s != 0u) return s;
-    if (wall_clock64() - t0 > 4 * kArriveTicks) {
+    if (wall_clock64() - t0 > 4ull * ticks) {
       const unsigned was = acas(&c->state, 0u, kResLate);
       return was != 0u ? was : kResLate;
     }
@@ -540,7 +536,8 @@ struct ResWave {
 
   __device__ __forceinline__ void run(const RveDev& r, const ResTile& q, int cur, VT* Vx, VT* Vy,
                                       int v, int nw, Lds& lds, int n, const char* xch,
-                                      unsigned xpar, unsigned tag0, bool& lost) {
+                                      unsigned xpar, unsigned tag0, unsigned pollLimit,
+                                      bool& lost) {
     const int nX = r.nX, nY = r.nY, sx = nX + 1;
     const int L = threadIdx.x & 63;
     const int i = q.s + L;
@@ -686,7 +683,7 @@ struct ResWave {
             if (rows) w.get(x, xi, xg, rs);
             const bool late = (cols && !c.is(tag)) || (rows && !w.is(tag));
             if (!__any(late)) break;
-            if (lost || polls >= kPollLimit) {
+            if (lost || polls >= pollLimit) {
               lost = true;
               break;
             }
@@ -813,7 +810,7 @@ template <typename CT, typename VT, int R, int T, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(res_waves<CT, R>()))) void k_resident(
     const RveDev* __restrict__ rves, const ResTile* __restrict__ tiles, int parity, int vpar,
     int n, const char* xch, unsigned xpar, unsigned tag0, ResCtl* ctl, unsigned cost,
-    unsigned cap, unsigned* told) {
+    unsigned cap, ResLimits lim, unsigned* told) {
   using Lds = ResLds<CT, VT, R, T, NW>;
   __shared__ Lds lds;
   const int v = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -827,7 +824,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(res_wav
       (&lds.zeroV[0][0][0])[2 * threadIdx.x + 1] = (VT)0;
     }
   }
-  if (threadIdx.x == 0) lds.state = res_arrive(ctl, gridDim.x, cost, cap);
+  if (threadIdx.x == 0) lds.state = res_arrive(ctl, gridDim.x, cost, cap, lim.arriveTicks);
   __syncthreads();
   if (lds.state == kResGo) {
     bool lost = false;
@@ -851,7 +848,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(res_wav
 #define EP2D_RES(EX, EY, CLEAN)                                                     \
   {                                                                                 \
     ResWave<CT, VT, R, T, NW, EX, EY, CLEAN> wv;                                    \
-    wv.run(r, q, cur, Vx, Vy, v, nw, lds, n, xch, xpar, tag0, lost);                \
+    wv.run(r, q, cur, Vx, Vy, v, nw, lds, n, xch, xpar, tag0, lim.polls, lost);                \
   }
       if (ex && clean) EP2D_RES(true, true, true)
       else if (ex) EP2D_RES(true, true, false)
@@ -967,10 +964,10 @@ void launch_resident(const ResLaunch& a, hipStream_t s, hipEvent_t e0, hipEvent_
     const char* xch = a.xch;
     if (e0)
       hipExtLaunchKernelGGL(kern, grid, block, 0, s, e0, e1, 0, a.rves, a.list, a.parity, a.vpar,
-                            a.iters, xch, a.xpar, a.tag0, a.ctl, a.cost, a.room, a.told);
+                            a.iters, xch, a.xpar, a.tag0, a.ctl, a.cost, a.room, a.limits, a.told);
     else
       hipLaunchKernelGGL(kern, grid, block, 0, s, a.rves, a.list, a.parity, a.vpar, a.iters, xch,
-                         a.xpar, a.tag0, a.ctl, a.cost, a.room, a.told);
+                         a.xpar, a.tag0, a.ctl, a.cost, a.room, a.limits, a.told);
     return 0;
   });
   EP2D_HIP(hipGetLastError());

@@ -467,6 +467,7 @@ void Solver::launchResidentRun(long n) {
   a.ctl = dResCtl_;
   a.cost = resCost_;
   a.room = resRoom_;
+  a.limits = resLimits_;
   a.told = hResTold_;
   *hResTold_ = 0;
   launch_resident(a, stream_, timed ? ev.first : nullptr, timed ? ev.second : nullptr);
@@ -490,9 +491,13 @@ bool Solver::settled() {
   const long n = resPending_;
   resPending_ = 0;
   const unsigned how = *hResTold_;
-  if (how == kResGo) return true;
-  if (how != kResNoRoom && how != kResLate)
-    throw HipError("a resident run lost a wait for a neighbouring tile");
+  if (how == kResGo) {
+    resCounts_[0]++;
+    return true;
+  }
+  const bool lost = how != kResNoRoom && how != kResLate;
+  resCounts_[lost ? 2 : 1]++;
+  if (lost) throw HipError("a resident run lost a wait for a neighbouring tile");
   if (how == kResLate) resSkip_ = 256;
   cur_ ^= 1;
   iterateLaunches(n);
@@ -505,6 +510,24 @@ void Solver::settle() {
   EP2D_HIP(hipSetDevice(device_));
   EP2D_HIP(hipStreamSynchronize(stream_));
   settled();
+}
+
+// Counts of the handle's resident runs (completed, turned away or late, lost),
+// and the bounds and exchange tag of its later ones (negative: unchanged).
+void Solver::diagResident(const long long* limits, long long* counts) {
+  settle();
+  for (int k = 0; counts && k < 3; k++) counts[k] = resCounts_[k];
+  if (!limits || resTiles_ == 0) return;
+  for (int k = 0; k < 3; k++)
+    if (limits[k] > 0xffffffffLL) throw ArgError("ep2d_diag_resident: limit out of range");
+  if (limits[0] >= 0) resLimits_.arriveTicks = (unsigned)limits[0];
+  if (limits[1] >= 0) resLimits_.polls = (unsigned)limits[1];
+  if (limits[2] >= 0) {
+    // (no word of the buffer carries a later tag)
+    EP2D_HIP(hipSetDevice(device_));
+    launch_fill((double*)dXch_, 2 * (size_t)resXpar_ / 8, 0.0, stream_);
+    resTag_ = (unsigned)limits[2];
+  }
 }
 
 Solver::~Solver() { release(); }

@@ -128,6 +128,7 @@ class Solver {
   void setTiming(long sampleEvery);
   void getTiming(double* avgMs, long* samples, const char** name);
   void sync();
+  void diagResident(const long long* limits, long long* counts);
   size_t deviceBytes() const { return devBytes_; }
 
  private:
@@ -197,6 +198,8 @@ class Solver {
   ResCtl* dResCtl_ = nullptr;
   unsigned* hResTold_ = nullptr;
   long resPending_ = 0;
+  ResLimits resLimits_;
+  long long resCounts_[3] = {0, 0, 0};  // completed, turned away or late, lost
   int resSkip_ = 0;                 // runs to take the other kernels after a late start
   void planResident(std::vector<ResTile>& tiles);
   bool residentFits(long n);

@@ -288,6 +288,17 @@ int ep2d_diag_copy(int device, size_t bytes, int reps, double* avgMs);
  * entries of four ints).  For tests of the order's coverage. */
 int ep2d_diag_chain_order(const int* segs, int n, int stageWaves, const int* dims, int nRves,
                           int resident, int* out, int outCapacity, int* nOut);
+/* Diagnostic, no counterpart in the reference: the resident runs of a handle
+ * (runs of 16 iterations and more of a grid that fits on the chip, in one
+ * launch).  counts (3 words, may be NULL) receives the runs completed, those
+ * whose workgroups could not all start (their iterations took the other
+ * kernels: the same results) and those that lost a wait inside the run.
+ * limits (3 words, may be NULL) sets, for the handle's later runs, [0] the
+ * ticks of 10 ns a launch waits for its workgroups (0: it never starts), [1]
+ * the polls of about a microsecond a wait inside the run takes, [2] the number
+ * its exchanges are counted on from (32 bits); negative: unchanged.  For tests
+ * of the paths a busy device takes. */
+int ep2d_diag_resident(ep2d_handle* h, const long long* limits, long long* counts);
 /* Analytic static solution of the single-pore problem beside the numerical
  * fields of the current state (SaveAnStatic2D, EffPlast2D.cu:1060-1292; the
  * reference calls it after ComputeEffModuli with nTasks > 1 and after

@@ -1,0 +1,103 @@
+"""Which path the iterations of a handle took: resident runs are counted by their
+outcome, so a run that was meant to be resident is seen to be one, and the paths
+a busy device takes are forced from the host (a launch that may not wait for its
+workgroups).  Every path gives the tile kernel's bits (no tolerance)."""
+import numpy as np
+import pytest
+# torch before the library: one HIP runtime in the process
+import torch  # noqa: F401
+
+from effplast2d_amd import EffPlast2D
+from tests.pairs import PLASTIC_FIELDS, STATE_FIELDS, STRESS_FIELDS, make_pa, random_state
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = STATE_FIELDS + STRESS_FIELDS + PLASTIC_FIELDS
+
+
+def _case(nX, mode, seed):
+    pa = make_pa(nX, nPores=1 + nX % 3, porosity=0.03)
+    init = random_state(nX, seed, pa=pa, boundary_v=True)
+    if mode == "split":
+        for k in ("Vx", "Vy"):
+            init[k] = init[k].astype(np.float32).astype(np.float64)
+    return pa, init
+
+
+def _start(g, init):
+    for k in STATE_FIELDS:
+        g.set(k, init[k])
+
+
+def _same(a, b):
+    for k in a:
+        assert np.array_equal(a[k], b[k], equal_nan=True), \
+            f"{k}: {np.count_nonzero(a[k] != b[k])} differ"
+
+
+def _tiles(nX, mode, pa, init, n):
+    with EffPlast2D(pa, nX, nTasks=3, mode=mode, tileRows=8) as g:
+        _start(g, init)
+        g.iterate(n)
+        return {k: g.get(k) for k in FIELDS}
+
+
+# the smallest and largest grid of each tile shape
+@pytest.mark.parametrize("mode,nX", [("fp64", 16), ("fp64", 333), ("fp64", 448), ("fp64", 560),
+                                     ("fp64", 672), ("fp64", 768), ("split", 16), ("split", 352),
+                                     ("split", 448), ("split", 560)])
+def test_long_runs_are_resident(mode, nX):
+    print(f"resident {mode} nX={nX}", flush=True)
+    pa, init = _case(nX, mode, 50 + nX)
+    with EffPlast2D(pa, nX, nTasks=3, mode=mode) as g:
+        _start(g, init)
+        for n in (16, 15, 40):      # the second takes the chains
+            g.iterate(n)
+        assert g.diag_resident() == (2, 0, 0)
+
+
+@pytest.mark.parametrize("mode,nX", [("fp64", 64), ("split", 333), ("fp64", 500)])
+def test_runs_that_may_not_start(mode, nX):
+    """A launch that finds no time for its workgroups leaves the state alone; its
+    iterations take the chains, and so do the runs after it."""
+    print(f"late start {mode} nX={nX}", flush=True)
+    pa, init = _case(nX, mode, 7 + nX)
+    with EffPlast2D(pa, nX, nTasks=3, mode=mode) as g:
+        _start(g, init)
+        g.diag_resident(arrive_ticks=0)
+        for n in (33, 16, 18):
+            g.iterate(n)
+        a = {k: g.get(k) for k in FIELDS}
+        assert g.diag_resident() == (0, 1, 0)
+    _same(a, _tiles(nX, mode, pa, init, 67))
+
+
+@pytest.mark.parametrize("mode", ["fp64", "split"])
+def test_runs_of_several_launches(mode):
+    """One call of more than 65536 iterations is several launches."""
+    nX, n = 17, 2 * 65536 + 21
+    print(f"long run {mode}", flush=True)
+    pa, init = _case(nX, mode, 3)
+    with EffPlast2D(pa, nX, nTasks=3, mode=mode) as g:
+        _start(g, init)
+        g.iterate(n)
+        a = {k: g.get(k) for k in FIELDS}
+        assert g.diag_resident() == (3, 0, 0)
+    _same(a, _tiles(nX, mode, pa, init, n))
+
+
+@pytest.mark.parametrize("mode", ["fp64", "split"])
+def test_exchange_numbers_start_again(mode):
+    """The 32 bits that count the exchanges run out: the buffer is cleared and
+    the count starts again."""
+    nX = 125
+    print(f"exchange numbers {mode}", flush=True)
+    pa, init = _case(nX, mode, 9)
+    with EffPlast2D(pa, nX, nTasks=3, mode=mode) as g:
+        _start(g, init)
+        g.diag_resident(tag=2 ** 32 - 1 - 150)
+        for n in (64, 64, 64, 64):
+            g.iterate(n)
+        a = {k: g.get(k) for k in FIELDS}
+        assert g.diag_resident() == (4, 0, 0)
+    _same(a, _tiles(nX, mode, pa, init, 256))
