@@ -1,7 +1,8 @@
-"""Which path the iterations of a handle took: resident runs are counted by their
-outcome, so a run that was meant to be resident is seen to be one, and the paths
-a busy device takes are forced from the host (a launch that may not wait for its
-workgroups).  Every path gives the tile kernel's bits (no tolerance)."""
+"""Which path the iterations of a handle on the automatic shape took: resident
+runs are counted by their outcome, so a run that was meant to be resident is
+seen to be one, and the paths a busy device takes are forced from the host (a
+launch that may not wait for its workgroups).  Every path gives the tile
+kernel's bits (no tolerance)."""
 import numpy as np
 import pytest
 # torch before the library: one HIP runtime in the process
@@ -42,10 +43,10 @@ def _tiles(nX, mode, pa, init, n):
         return {k: g.get(k) for k in FIELDS}
 
 
-# the smallest and largest grid of each tile shape
-@pytest.mark.parametrize("mode,nX", [("fp64", 16), ("fp64", 333), ("fp64", 448), ("fp64", 560),
-                                     ("fp64", 672), ("fp64", 768), ("split", 16), ("split", 352),
-                                     ("split", 448), ("split", 560)])
+# the smallest and largest grid of each tile shape, on 256 CUs
+@pytest.mark.parametrize("mode,nX", [("fp64", 16), ("fp64", 336), ("fp64", 448), ("fp64", 560),
+                                     ("fp64", 672), ("fp64", 792), ("split", 16), ("split", 448),
+                                     ("split", 449), ("split", 560)])
 def test_long_runs_are_resident(mode, nX):
     print(f"resident {mode} nX={nX}", flush=True)
     pa, init = _case(nX, mode, 50 + nX)
@@ -101,3 +102,23 @@ def test_exchange_numbers_start_again(mode):
         a = {k: g.get(k) for k in FIELDS}
         assert g.diag_resident() == (4, 0, 0)
     _same(a, _tiles(nX, mode, pa, init, 256))
+
+
+# grids below 16, between and beyond the resident shapes' ranges, up to the
+# largest that takes the shortest segments of one round
+@pytest.mark.parametrize("mode,nX", [(m, n) for m in ("fp64", "split") for n in (8, 9, 15)] +
+                         [("fp64", n) for n in (337, 447, 561, 671, 793, 900, 1023, 1024)] +
+                         [("split", n) for n in (561, 700, 900, 1023, 1024)])
+def test_automatic_chains_equal_tiles(mode, nX):
+    """Without a resident shape the automatic shape is a chain on segments of a
+    computed height, with closing launches of as few rows."""
+    print(f"automatic chains {mode} nX={nX}", flush=True)
+    pa, init = _case(nX, mode, 11 + nX)
+    steps = (21, 4, 3, 2, 1, 16)
+    with EffPlast2D(pa, nX, nTasks=3, mode=mode) as g:
+        _start(g, init)
+        for n in steps:
+            g.iterate(n)
+        a = {k: g.get(k) for k in FIELDS}
+        assert g.diag_resident() == (0, 0, 0)
+    _same(a, _tiles(nX, mode, pa, init, sum(steps)))
