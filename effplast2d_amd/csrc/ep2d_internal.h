@@ -183,9 +183,10 @@ void launch_wide(int ns, const RveDev* rves, const int4* segs, int nsegs, int pa
 // ---- resident runs (ep2d_resident.hip) ---------------------------------------
 // Shape of a tile's workgroup: waves of `rows` rows each (64 columns), and the
 // iterations between two exchanges with the neighbouring tiles.
-// cost: half CUs a tile is given (2: one tile to a CU); from: smallest grid.
+// cost: half CUs a tile is given (2: one tile to a CU); from, to: smallest and
+// largest grid (to 0: as long as the tiles find room).
 struct ResShape {
-  int rows = 0, every = 1, waves = 8, cost = 2, from = 0;
+  int rows = 0, every = 1, waves = 8, cost = 2, from = 0, to = 0;
 };
 // One tile: own columns [i0, i1) and rows [j0, j1) of RVE rve; lane 0 is
 // column s, the first wave's first row is jr.  xl, xr, xu, xd: places of its

@@ -895,26 +895,29 @@ int res_parts(int n, int span, int T) {
 }  // namespace
 
 // From runs of 500 iterations of one RVE whose nodes yield (us per iteration; in
-// brackets the chains on the shortest segments of one round):
-//   split, two rows a wave:  64^2 2.6 (3.1), 256^2 2.6 (3.3), 333^2 3.0 (3.9),
-//     with two tiles to a CU 352^2 3.4 (3.9)
-//   split, four rows, one tile to a CU:  400^2 4.1 (4.0), 450^2 4.2 (4.3), 512^2
-//     3.9 (4.3), 560^2 4.1 (4.5); with two tiles to a CU the chains were faster
-//   FP64, two rows:  64^2 4.1 (4.7), 256^2 4.0 (5.4), 333^2 4.2 (5.8)
-//   FP64, four rows:  352^2 6.2 (5.9), 400^2 6.3 (6.3), 450^2 6.4 (6.5), 512^2
-//     6.2 (6.9), 560^2 6.2 (7.2)
-//   FP64, six rows, an exchange each iteration:  672^2 8.2 (8.3), 700^2 8.0 (8.4),
-//     768^2 8.3 (9.2); beyond, the tiles find no room.  600^2 and 640^2 lie past
-//     the four rows' room: chains, 7.5
+// brackets the chains on the shortest segments of one round, at the same size
+// in the same process):
+//   split, two rows a wave:  64^2 2.6 (3.1), 256^2 2.6 (3.3), 336^2 3.1 (3.8),
+//     with two tiles to a CU 352^2 3.4 (3.8), 392^2 3.5 (3.9); with eight strips
+//     from 393^2 on 4.2 (3.9) and 447^2 4.7 (4.0): chains up to 447^2
+//   split, four rows, one tile to a CU:  449^2 4.15 (4.12), 480^2 4.15 (4.04),
+//     505^2 3.9 (4.1), 512^2 3.9 (4.1), 560^2 4.1 (4.3)
+//   FP64, two rows:  64^2 4.0 (4.8), 256^2 4.1 (5.4), 336^2 4.2 (5.8); from 337^2
+//     on the tiles find no room
+//   FP64, four rows:  352^2 6.2 (5.9), 400^2 6.3 (6.3), 448^2 6.3 (6.6), 504^2
+//     6.5 (6.5), 512^2 6.1 (6.7), 560^2 6.2 (7.2)
+//   FP64, six rows, an exchange each iteration:  672^2 8.3 (8.3), 700^2 8.2 (8.4),
+//     768^2 8.4 (9.1), 792^2 8.3 (9.4); from 793^2 on the tiles find no room.
+//     600^2 and 640^2 lie past the four rows' room: chains, 7.5
 std::vector<ResShape> resident_shapes(int mode) {
-  if (mode == 2) return {{2, 2, 8, 1, 0}, {4, 2, 8, 2, 448}};
+  if (mode == 2) return {{2, 2, 8, 1, 0, 392}, {4, 2, 8, 2, 448}};
   return {{2, 2, 8, 2, 0}, {4, 2, 8, 2, 448}, {6, 1, 8, 2, 672}};
 }
 
 int resident_tiles(const ResShape& sh, int mode, int n, int rve, size_t x0, ResTile* out,
                    size_t* pairs) {
   const int T = sh.every, H = sh.rows * sh.waves;
-  if (H <= 4 * T || n < sh.from) return 0;
+  if (H <= 4 * T || n < sh.from || (sh.to > 0 && n > sh.to)) return 0;
   const int strips = res_parts(n, 64, T), bands = res_parts(n, H, T);
   // a tile's own part is at least as wide as what its neighbours read of it
   if ((strips > 1 && n / strips < 4 * T) || (bands > 1 && n / bands < 2 * T)) return 0;

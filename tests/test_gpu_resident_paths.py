@@ -45,8 +45,8 @@ def _tiles(nX, mode, pa, init, n):
 
 # the smallest and largest grid of each tile shape, on 256 CUs
 @pytest.mark.parametrize("mode,nX", [("fp64", 16), ("fp64", 336), ("fp64", 448), ("fp64", 560),
-                                     ("fp64", 672), ("fp64", 792), ("split", 16), ("split", 448),
-                                     ("split", 449), ("split", 560)])
+                                     ("fp64", 672), ("fp64", 792), ("split", 16), ("split", 392),
+                                     ("split", 448), ("split", 560)])
 def test_long_runs_are_resident(mode, nX):
     print(f"resident {mode} nX={nX}", flush=True)
     pa, init = _case(nX, mode, 50 + nX)
@@ -108,7 +108,7 @@ def test_exchange_numbers_start_again(mode):
 # largest that takes the shortest segments of one round
 @pytest.mark.parametrize("mode,nX", [(m, n) for m in ("fp64", "split") for n in (8, 9, 15)] +
                          [("fp64", n) for n in (337, 447, 561, 671, 793, 900, 1023, 1024)] +
-                         [("split", n) for n in (561, 700, 900, 1023, 1024)])
+                         [("split", n) for n in (393, 447, 561, 700, 900, 1023, 1024)])
 def test_automatic_chains_equal_tiles(mode, nX):
     """Without a resident shape the automatic shape is a chain on segments of a
     computed height, with closing launches of as few rows."""
