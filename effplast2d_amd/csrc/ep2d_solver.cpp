@@ -428,6 +428,7 @@ void Solver::planResident(std::vector<ResTile>& tiles) {
     resXpar_ = (unsigned)((pairs * 16 + 255) / 256 * 256);
     resTiles_ = n;
     hResTold_ = (unsigned*)(hMax_ + 3);  // the word past the residual's three
+    lastResident_ = true;
     return;
   }
 }
@@ -475,12 +476,10 @@ void Solver::launchResidentRun(long n) {
   resPending_ = n;
   cur_ ^= 1;
   stressStale_ = true;
-  if (timed) {
-    pending_.push_back(ev);
-    pendingIters_.push_back((int)n);
-    if (pending_.size() >= 256) resolveTiming(false);
-  }
+  // (the newest samples stay unread until the run's outcome is known)
+  if (timed) noteTimed(ev, kTimedResident, n);
   launchCount_++;
+  lastResident_ = true;
 }
 
 // Outcome of the last resident run, the stream being idle: true when there
@@ -494,6 +493,11 @@ bool Solver::settled() {
   if (how == kResGo) {
     resCounts_[0]++;
     return true;
+  }
+  // the launch computed nothing: its duration is no sample
+  if (!pending_.empty() && pending_.back().kind == kTimedResident) {
+    freeEvents_.push_back(pending_.back().ev);
+    pending_.pop_back();
   }
   const bool lost = how != kResNoRoom && how != kResLate;
   resCounts_[lost ? 2 : 1]++;
@@ -537,16 +541,12 @@ void Solver::release() {
   (void)hipSetDevice(device_);
   if (stream_) (void)hipStreamSynchronize(stream_);
   dropPlainGraph();
-  for (auto& e : pending_) {
-    (void)hipEventDestroy(e.first);
-    (void)hipEventDestroy(e.second);
-  }
+  for (auto& p : pending_) freeEvents_.push_back(p.ev);
   for (auto& e : freeEvents_) {
     (void)hipEventDestroy(e.first);
     (void)hipEventDestroy(e.second);
   }
   pending_.clear();
-  pendingIters_.clear();
   freeEvents_.clear();
   // the stream is idle: the blocks can go back to the pool
   for (auto& a : allocs_) {
@@ -676,16 +676,7 @@ void Solver::launchIteration() {
   const bool plastic = opt_.nTasks > 1;   // EffPlast2D.cu:392
   const bool timed = sampleEvery_ > 0 && (launchCount_ % sampleEvery_) == 0;
   std::pair<hipEvent_t, hipEvent_t> ev{};
-  if (timed) {
-    if (freeEvents_.empty()) {
-      hipEvent_t a, b;
-      EP2D_HIP(hipEventCreate(&a));
-      EP2D_HIP(hipEventCreate(&b));
-      freeEvents_.push_back({a, b});
-    }
-    ev = freeEvents_.back();
-    freeEvents_.pop_back();
-  }
+  if (timed) ev = takeTimingEvents();
   // timed launches carry their own start/stop events (hipExtLaunchKernelGGL),
   // which record the dispatch's execution window
   if (mode_ == EP2D_MODE_PLAIN) {
@@ -713,11 +704,7 @@ void Solver::launchIteration() {
     cur_ ^= 1;
     stressStale_ = true;
   }
-  if (timed) {
-    pending_.push_back(ev);
-    pendingIters_.push_back(1);
-    if (pending_.size() >= 256) resolveTiming(false);
-  }
+  if (timed) noteTimed(ev, kTimedSingle, 1);
   launchCount_++;
 }
 
@@ -731,6 +718,11 @@ std::pair<hipEvent_t, hipEvent_t> Solver::takeTimingEvents() {
   auto ev = freeEvents_.back();
   freeEvents_.pop_back();
   return ev;
+}
+
+void Solver::noteTimed(const std::pair<hipEvent_t, hipEvent_t>& ev, TimedKind kind, long iters) {
+  pending_.push_back({ev, kind, iters});
+  if (pending_.size() >= 256) resolveTiming(false);
 }
 
 // ipl_ iterations in one launch (each segment on a pair of waves or a chain
@@ -752,11 +744,7 @@ void Solver::launchMulti(int q) {
                  timed ? ev.first : nullptr, timed ? ev.second : nullptr, stageWaves_);
   cur_ ^= 1;
   stressStale_ = true;
-  if (timed) {
-    pending_.push_back(ev);
-    pendingIters_.push_back(ipl_);
-    if (pending_.size() >= 256) resolveTiming(false);
-  }
+  if (timed) noteTimed(ev, kTimedMulti, ipl_);
   launchCount_++;
 }
 
@@ -837,6 +825,7 @@ void Solver::dropPlainGraph() {
 }
 
 void Solver::iterateLaunches(long n) {
+  if (n > 0) lastResident_ = false;
   n -= replayPlain(n);
   if (!multiIter_ || (stress64_ && !multi64())) {
     for (long k = 0; k < n; k++) launchIteration();
@@ -881,16 +870,15 @@ void Solver::launchClose(int ns, int q) {
 void Solver::resolveTiming(bool all) {
   const size_t keep = all ? 0 : 64;
   while (pending_.size() > keep) {
-    auto ev = pending_.front();
-    const int its = pendingIters_.front();
+    const TimedLaunch p = pending_.front();
     pending_.erase(pending_.begin());
-    pendingIters_.erase(pendingIters_.begin());
-    EP2D_HIP(hipEventSynchronize(ev.second));
+    freeEvents_.push_back(p.ev);
+    EP2D_HIP(hipEventSynchronize(p.ev.second));
     float ms = 0.f;
-    EP2D_HIP(hipEventElapsedTime(&ms, ev.first, ev.second));
+    EP2D_HIP(hipEventElapsedTime(&ms, p.ev.first, p.ev.second));
     timedMs_ += ms;          // averages are per iteration
-    timedSamples_ += its;
-    freeEvents_.push_back(ev);
+    timedSamples_ += p.iters;
+    timedOf_[p.kind] += p.iters;
   }
 }
 
@@ -900,6 +888,7 @@ void Solver::setTiming(long sampleEvery) {
   sampleEvery_ = sampleEvery < 0 ? 0 : sampleEvery;
   timedMs_ = 0.0;
   timedSamples_ = 0;
+  for (long& t : timedOf_) t = 0;
   launchCount_ = 0;
 }
 
@@ -909,34 +898,41 @@ void Solver::getTiming(double* avgMs, long* samples, const char** name) {
   if (avgMs) *avgMs = timedSamples_ ? timedMs_ / timedSamples_ : 0.0;
   if (samples) *samples = timedSamples_;
   if (name) {
+    // the kernel most of the samples are of; without samples, the one the last
+    // iterations took
+    int k = lastResident_ ? kTimedResident : multiIter_ ? kTimedMulti : kTimedSingle;
+    if (timedSamples_ > 0)
+      k = (int)(std::max_element(timedOf_, timedOf_ + kTimedKinds) - timedOf_);
     // held by the handle: the pointer stays valid until the next call or
     // the handle's destruction
-    std::string& nm = timingName_;
-    nm = fused_kernel_name(mode_);
-    if (resTiles_ > 0)
-      nm = std::string(mode_ == EP2D_MODE_SPLIT ? "k_resident<float, float, "
-                                                : "k_resident<double, double, ") +
+    timingName_ = kernelName((TimedKind)k);
+    *name = timingName_.c_str();
+  }
+}
+
+std::string Solver::kernelName(TimedKind kind) const {
+  const bool f32 = mode_ == EP2D_MODE_SPLIT;
+  if (kind == kTimedResident)
+    return std::string(f32 ? "k_resident<float, float, " : "k_resident<double, double, ") +
            std::to_string(resShape_.rows) + ", " + std::to_string(resShape_.every) + ", " +
-           std::to_string(resShape_.waves) + "> tiles=" + std::to_string(resTiles_) + " (per iteration)";
-    else if (marchRows_ > 0 && multiIter_)
-      nm = (ipl_ == 2 ? std::string(mode_ == EP2D_MODE_SPLIT ? "k_march2p<float, float>"
-                                                              : "k_march2p<double, double>")
+           std::to_string(resShape_.waves) + "> tiles=" + std::to_string(resTiles_) +
+           " (per iteration)";
+  if (kind == kTimedMulti)
+    return (ipl_ == 2 ? std::string(f32 ? "k_march2p<float, float>" : "k_march2p<double, double>")
             : wide_ ? "k_wide<" + std::to_string(ipl_) + ">"
-                    : std::string(mode_ == EP2D_MODE_SPLIT ? "k_chain<float, float, "
-                                                           : "k_chain<double, double, ") +
+                    : std::string(f32 ? "k_chain<float, float, " : "k_chain<double, double, ") +
                           std::to_string(ipl_) + ", " + std::to_string(stageWaves_) + ">") +
            " rows=" + std::to_string(marchRows_) + " segments=" + std::to_string(nSegs2_) +
            " (per iteration)";
-    else if (marchRows_ > 0)
-      nm = std::string(mode_ == EP2D_MODE_SPLIT ? "k_march<float, float>" : "k_march<double, double>") +
+  if (marchRows_ > 0 && !tileSingles_)
+    return std::string(f32 ? "k_march<float, float>" : "k_march<double, double>") +
            " rows=" + std::to_string(marchRows_) + " segments=" + std::to_string(nSegs_);
-    else if (mode_ != EP2D_MODE_PLAIN) nm += " TY=" + std::to_string(fplan_.ty) + " grid=" +
-                                        std::to_string(fplan_.grid) + " tiles=" +
-                                        std::to_string(fplan_.ntiles) + " waves=" +
-                                        std::to_string(fplan_.waves) + " blocks/CU=" +
-                                        std::to_string(fplan_.blocksPerCU);
-    *name = nm.c_str();
-  }
+  std::string nm = fused_kernel_name(mode_);
+  if (mode_ != EP2D_MODE_PLAIN)
+    nm += " TY=" + std::to_string(fplan_.ty) + " grid=" + std::to_string(fplan_.grid) +
+          " tiles=" + std::to_string(fplan_.ntiles) + " waves=" + std::to_string(fplan_.waves) +
+          " blocks/CU=" + std::to_string(fplan_.blocksPerCU);
+  return nm;
 }
 
 void Solver::sync() {

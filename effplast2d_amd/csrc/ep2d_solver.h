@@ -215,7 +215,6 @@ class Solver {
   long plainIters_ = 0;             // iterations asked for so far
   long replayPlain(long n);
   void dropPlainGraph();
-  std::pair<hipEvent_t, hipEvent_t> takeTimingEvents();
   void launchMulti(int q);         // ipl_ iterations, q-th such launch of a run
   void launchClose(int ns, int q);  // ns = 3 or 2 iterations closing a run
   bool multi64() const;            // the FP64 finish runs on the multi-iteration shape
@@ -247,10 +246,21 @@ class Solver {
   // timing
   long sampleEvery_ = 0;
   long launchCount_ = 0;
-  std::vector<std::pair<hipEvent_t, hipEvent_t>> pending_, freeEvents_;
-  std::vector<int> pendingIters_;   // iterations in each pending timed launch
+  enum TimedKind { kTimedSingle, kTimedMulti, kTimedResident, kTimedKinds };
+  struct TimedLaunch {
+    std::pair<hipEvent_t, hipEvent_t> ev;
+    TimedKind kind;
+    long iters;
+  };
+  std::vector<TimedLaunch> pending_;   // sampled launches not read yet
+  std::vector<std::pair<hipEvent_t, hipEvent_t>> freeEvents_;
   double timedMs_ = 0.0;
   long timedSamples_ = 0;
+  long timedOf_[kTimedKinds] = {0};  // the samples by kernel
+  bool lastResident_ = false;        // the last iterations ran resident
+  std::pair<hipEvent_t, hipEvent_t> takeTimingEvents();
+  void noteTimed(const std::pair<hipEvent_t, hipEvent_t>& ev, TimedKind kind, long iters);
+  std::string kernelName(TimedKind kind) const;
   std::string timingName_;         // kernel name getTiming() hands out
 
   // job state

@@ -268,7 +268,9 @@ int ep2d_hole_area(ep2d_handle* h, ep2d_record* rec);
 
 /* ---- timing ----------------------------------------------------------------
  * Sample the duration of the dominant iteration kernel with HIP events on
- * the handle's stream: every sampleEvery-th launch is bracketed (0: off). */
+ * the handle's stream: every sampleEvery-th launch is bracketed (0: off).  A
+ * launch of n iterations is n samples; kernelName is the kernel most samples
+ * are of (without samples, the one the last iterations took). */
 int ep2d_set_timing(ep2d_handle* h, long sampleEvery);
 int ep2d_get_timing(ep2d_handle* h, double* avgKernelMs, long* samples,
                     const char** kernelName);

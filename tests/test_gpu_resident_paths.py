@@ -122,3 +122,33 @@ def test_automatic_chains_equal_tiles(mode, nX):
         a = {k: g.get(k) for k in FIELDS}
         assert g.diag_resident() == (0, 0, 0)
     _same(a, _tiles(nX, mode, pa, init, sum(steps)))
+
+
+@pytest.mark.parametrize("mode,nX", [("fp64", 500), ("split", 500)])
+def test_a_run_that_did_not_start_is_no_sample(mode, nX):
+    """Its iterations are timed where they ran, on the chains: as many samples
+    as a run on the chains gives, and their name."""
+    print(f"timing of a late start {mode}", flush=True)
+    pa, init = _case(nX, mode, 21)
+
+    def run(n, calls, late):
+        with EffPlast2D(pa, nX, nTasks=3, mode=mode) as g:
+            _start(g, init)
+            if late:
+                g.diag_resident(arrive_ticks=0)
+            g.set_timing(1)
+            for _ in range(calls):
+                g.iterate(n)
+            return g.timing()
+
+    # 401 iterations: 100 four-iteration launches and one on its own
+    ms, n, name = run(401, 1, True)
+    assert n == 401 and "k_chain" in name, (ms, n, name)
+    ms, n, name = run(401, 3, False)
+    assert n == 3 * 401 and "k_resident" in name, (ms, n, name)
+    # short runs: 3 four-iteration launches, a closing one of two (not
+    # sampled) and one on its own
+    ms, n, name = run(15, 2, False)
+    assert n == 2 * 13 and "k_chain" in name, (ms, n, name)
+    ms, n, name = run(1, 3, False)
+    assert n == 3 and "k_fused" in name, (ms, n, name)
