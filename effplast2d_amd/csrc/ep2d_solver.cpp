@@ -501,25 +501,47 @@ bool Solver::settled() {
   }
   const bool lost = how != kResNoRoom && how != kResLate;
   resCounts_[lost ? 2 : 1]++;
-  if (lost) throw HipError("a resident run lost a wait for a neighbouring tile");
-  if (how == kResLate) resSkip_ = 256;
+  if (lost || how == kResLate) resSkip_ = 256;
+  if (lost) {
+    // U and V are torn: no call uses them until they are set again (the
+    // stress fields are as in a new handle)
+    lostFields_ = 15;
+    const size_t nC = (size_t)nX_ * nY_, nV = (size_t)(nX_ - 1) * (nY_ - 1);
+    for (double* p : {f_.P, f_.tauXX, f_.tauYY, f_.tauXYav, f_.J2})
+      launch_fill(p, nC, 0.0, stream_);
+    for (double* p : {f_.tauXY, f_.J2XY}) launch_fill(p, nV, 0.0, stream_);
+    stressStale_ = false;
+    throw HipError("a resident run lost a wait for a neighbouring tile");
+  }
   cur_ ^= 1;
   iterateLaunches(n);
   return false;
 }
 
-// Before anything that uses the state: a resident run's outcome is known.
-void Solver::settle() {
+// A resident run's outcome is known.
+void Solver::settleRun() {
   if (resPending_ == 0) return;
   EP2D_HIP(hipSetDevice(device_));
   EP2D_HIP(hipStreamSynchronize(stream_));
   settled();
 }
 
+void Solver::requireState() const {
+  if (lostFields_)
+    throw StatusError(EP2D_ERR_STATE,
+                      "U and V are not valid after a lost resident run: set Ux, Uy, Vx and Vy");
+}
+
+// Before anything that uses the state.
+void Solver::settle() {
+  settleRun();
+  requireState();
+}
+
 // Counts of the handle's resident runs (completed, turned away or late, lost),
 // and the bounds and exchange tag of its later ones (negative: unchanged).
 void Solver::diagResident(const long long* limits, long long* counts) {
-  settle();
+  settleRun();
   for (int k = 0; counts && k < 3; k++) counts[k] = resCounts_[k];
   if (!limits || resTiles_ == 0) return;
   for (int k = 0; k < 3; k++)
@@ -883,7 +905,7 @@ void Solver::resolveTiming(bool all) {
 }
 
 void Solver::setTiming(long sampleEvery) {
-  settle();
+  settleRun();
   resolveTiming(true);
   sampleEvery_ = sampleEvery < 0 ? 0 : sampleEvery;
   timedMs_ = 0.0;
@@ -893,7 +915,7 @@ void Solver::setTiming(long sampleEvery) {
 }
 
 void Solver::getTiming(double* avgMs, long* samples, const char** name) {
-  settle();
+  settleRun();
   resolveTiming(true);
   if (avgMs) *avgMs = timedSamples_ ? timedMs_ / timedSamples_ : 0.0;
   if (samples) *samples = timedSamples_;
@@ -936,7 +958,7 @@ std::string Solver::kernelName(TimedKind kind) const {
 }
 
 void Solver::sync() {
-  settle();
+  settleRun();
   EP2D_HIP(hipStreamSynchronize(stream_));
 }
 
@@ -962,6 +984,7 @@ void Solver::applyAffine(double dUxdx, double dUydy, double dUxdy, double dUydx)
 
 // EffPlast2D.cu:407-412 (step-level entry point).
 double Solver::residual(const double e[3], long* nonfinite) {
+  requireState();
   // (a resident run that did not start is made up for, and the residual taken
   // again)
   do {
@@ -1667,10 +1690,10 @@ void Solver::setField(int field, const double* host, size_t count) {
   const size_t N = (size_t)m * n;
   if (count < N) throw ArgError("host buffer too small for field");
   EP2D_HIP(hipSetDevice(device_));
-  settle();
+  settleRun();
   switch (field) {
-    case EP2D_FIELD_UX: h2d(r_.Ux[cur_], host, N); return;
-    case EP2D_FIELD_UY: h2d(r_.Uy[cur_], host, N); return;
+    case EP2D_FIELD_UX: h2d(r_.Ux[cur_], host, N); lostFields_ &= ~1u; return;
+    case EP2D_FIELD_UY: h2d(r_.Uy[cur_], host, N); lostFields_ &= ~2u; return;
     case EP2D_FIELD_VX: case EP2D_FIELD_VY: {
       // both buffers, so the velocities multi-iteration launches never write
       // (the boundary) agree
@@ -1683,6 +1706,7 @@ void Solver::setField(int field, const double* host, size_t count) {
       } else {
         for (int k = 0; k < nb; k++) h2d((double*)dst[k], host, N);
       }
+      lostFields_ &= field == EP2D_FIELD_VX ? ~4u : ~8u;
       return;
     }
     default:

@@ -205,7 +205,12 @@ class Solver {
   bool residentFits(long n);
   void launchResidentRun(long n);
   bool settled();                   // after the stream is synchronised
+  void settleRun();
   void settle();
+  // state fields (bits: Ux, Uy, Vx, Vy) a lost run left invalid and nobody has
+  // set since
+  unsigned lostFields_ = 0;
+  void requireState() const;
   void iterateLaunches(long n);
   // a run of plain iterations as a graph (replayPlain), and the RVE record its
   // launches were captured with

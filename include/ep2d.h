@@ -295,6 +295,8 @@ int ep2d_diag_chain_order(const int* segs, int n, int stageWaves, const int* dim
  * launch).  counts (3 words, may be NULL) receives the runs completed, those
  * whose workgroups could not all start (their iterations took the other
  * kernels: the same results) and those that lost a wait inside the run.
+ * After a lost one (reported once as EP2D_ERR_HIP) the calls that use the state
+ * return EP2D_ERR_STATE until Ux, Uy, Vx and Vy have been set.
  * limits (3 words, may be NULL) sets, for the handle's later runs, [0] the
  * ticks of 10 ns a launch waits for its workgroups (0: it never starts), [1]
  * the polls of about a microsecond a wait inside the run takes, [2] the number

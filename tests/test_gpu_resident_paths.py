@@ -8,7 +8,7 @@ import pytest
 # torch before the library: one HIP runtime in the process
 import torch  # noqa: F401
 
-from effplast2d_amd import EffPlast2D
+from effplast2d_amd import EffPlast2D, Ep2dError
 from tests.pairs import PLASTIC_FIELDS, STATE_FIELDS, STRESS_FIELDS, make_pa, random_state
 
 pytestmark = pytest.mark.gpu
@@ -152,3 +152,35 @@ def test_a_run_that_did_not_start_is_no_sample(mode, nX):
     assert n == 2 * 13 and "k_chain" in name, (ms, n, name)
     ms, n, name = run(1, 3, False)
     assert n == 3 and "k_fused" in name, (ms, n, name)
+
+
+@pytest.mark.parametrize("mode", ["fp64", "split"])
+def test_a_lost_run_leaves_no_state(mode):
+    """A run that lost a wait (here: one that may not wait for its neighbours'
+    words) is reported, and nothing reads its torn fields: every call that uses
+    the state fails until U and V are set, then the handle goes on."""
+    nX = 200
+    print(f"lost run {mode}", flush=True)
+    pa, init = _case(nX, mode, 13)
+    with EffPlast2D(pa, nX, nTasks=3, mode=mode) as g:
+        _start(g, init)
+        g.diag_resident(polls=0)
+        g.iterate(2000)
+        with pytest.raises(Ep2dError) as e:
+            g.get("Ux")
+        assert e.value.status == -2         # EP2D_ERR_HIP
+        assert g.diag_resident(polls=1 << 20) == (0, 0, 1)
+        calls = [lambda: g.get("Ux"), lambda: g.get("tauXX"), lambda: g.iterate(1),
+                 lambda: g.iterate(100), lambda: g.residual([1e-3, 0.0, 0.0]),
+                 lambda: g.apply_affine(1e-3, 0.0, 0.0, 0.0), g.averages, g.boundary,
+                 g.hole_area, lambda: g.device_ptr("Vx"),
+                 lambda: g.ComputeEffModuli(-1e-3, [1.0, 1.0, 0.0])]
+        for k in STATE_FIELDS:
+            for c in calls:
+                with pytest.raises(Ep2dError) as e:
+                    c()
+                assert e.value.status == -7     # EP2D_ERR_STATE
+            g.set(k, init[k])
+        g.iterate(41)
+        a = {k: g.get(k) for k in FIELDS}
+    _same(a, _tiles(nX, mode, pa, init, 41))
