@@ -790,16 +790,15 @@ int Solver::iterMode() const { return stress64_ ? kModeSplitStress64 : mode_; }
 void Solver::iterate(long n) {
   EP2D_HIP(hipSetDevice(device_));
   settle();
-  if (residentFits(n)) {
-    // (a launch of a second at most, which other handles' work may wait for)
-    constexpr long kMost = 1L << 16;
-    for (; n > kMost; n -= kMost) {
-      launchResidentRun(kMost);
-      settle();
-    }
-    if (n >= kResMinIters) launchResidentRun(n);
-    else iterateLaunches(n);
-    return;
+  // (a launch of a second at most, which other handles' work may wait for; what
+  // follows one that started late takes the other kernels)
+  constexpr long kMost = 1L << 16;
+  while (residentFits(n)) {
+    const long m = std::min(n, kMost);
+    launchResidentRun(m);
+    n -= m;
+    if (n == 0) return;
+    settle();
   }
   iterateLaunches(n);
 }

@@ -184,3 +184,17 @@ def test_a_lost_run_leaves_no_state(mode):
         g.iterate(41)
         a = {k: g.get(k) for k in FIELDS}
     _same(a, _tiles(nX, mode, pa, init, 41))
+
+
+def test_one_late_start_a_call():
+    """The later launches of a call do not wait where the first one did in vain."""
+    nX, n = 40, 3 * 65536 + 20
+    print("late start of a long call", flush=True)
+    pa, init = _case(nX, "split", 5)
+    with EffPlast2D(pa, nX, nTasks=3, mode="split") as g:
+        _start(g, init)
+        g.diag_resident(arrive_ticks=0)
+        g.iterate(n)
+        a = {k: g.get(k) for k in FIELDS}
+        assert g.diag_resident() == (0, 1, 0)
+    _same(a, _tiles(nX, "split", pa, init, n))
