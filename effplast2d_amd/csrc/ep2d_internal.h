@@ -202,16 +202,16 @@ struct ResTile {
 struct ResCtl {
   unsigned arrive, state, depart, pad;
 };
-// Bounds of a launch's waits: for its other tiles (ticks of 10 ns; 0: it is
-// turned away at once) and for the words of one exchange (polls of about a
+// Bounds of a launch's waits: for its other tiles (ticks of 10 ns; 0: it does not
+// start) and for the words of one exchange (polls of about a
 // microsecond).
 struct ResLimits {
   unsigned arriveTicks = 25000000u, polls = 1u << 20;
 };
-// how a launch went: run, or ended with the fields untouched because other
-// launches hold the GPU's room or its tiles did not all start in time; lost:
-// a wait inside the run ended at its bound (the fields are not valid)
-constexpr unsigned kResGo = 1, kResNoRoom = 2, kResLate = 3, kResLost = 4;
+// how a launch went: run, or ended with the fields untouched because its tiles
+// did not all start in time; lost: a wait inside the run ended at its bound
+// (the fields are not valid)
+constexpr unsigned kResGo = 1, kResLate = 2, kResLost = 3;
 constexpr long kResMinIters = 16;  // shorter runs take the other kernels
 constexpr int kResMinSide = 16;
 struct ResLaunch {
@@ -226,9 +226,9 @@ struct ResLaunch {
   unsigned xpar;
   unsigned tag0;            // tags tag0 + 1 .. tag0 + iters, none used before
   ResCtl* ctl;
-  unsigned cost, room;      // half CUs of a tile, and of the device
   ResLimits limits;
-  unsigned* told;           // pinned host word that receives how the launch went
+  unsigned run;             // the number the launch is known by (not 0)
+  unsigned* told;           // two pinned host words: receive `run` if it ran, else how it failed
 };
 // The shapes of a scheme, from the smallest tiles to the largest: a grid takes
 // the first whose tiles find room together.
@@ -238,7 +238,7 @@ std::vector<ResShape> resident_shapes(int mode);
 // pairs of one half the RVE's edges take.
 int resident_tiles(const ResShape& sh, int mode, int n, int rve, size_t x0, ResTile* out,
                    size_t* pairs);
-int resident_room(int device);                        // half CUs
+int device_cus(int device);
 int resident_cost(const ResShape& sh, int mode);      // half CUs of a tile (0: does not fit)
 // `iters` iterations of every RVE of the list: U[cur] receives U before the
 // last iteration, U[cur ^ 1] U after it, V is updated in place.

@@ -33,14 +33,15 @@
 // hence read k-1's (all its waves: a barrier stands between).
 //
 // Every wait ends.  A tile waits for its neighbours, so all tiles of a launch
-// must run at once.  The first workgroup of a launch to run reserves room for
-// all of them in a per-device count of the tiles in flight (two to a CU: a
-// tile takes at most half of a CU's registers, LDS and waves, so any number of
-// launches whose tiles stay within the count find room), and no tile starts
-// before all have arrived.  If the room is taken (another handle's run) or
-// the tiles have not all arrived within a quarter second (another process
-// holds the GPU), the launch ends without having changed anything and says so,
-// and the caller takes the other kernels.  Waits inside the run are bounded too.
+// must run at once, and no tile starts before all have arrived.  The host lets
+// only so many launches of this process in as find their places together
+// (DeviceRoom): tiles of the split two-row shape take half a CU's registers (118
+// a lane at eight waves), the others (146 to 204) a CU each.  Other work on the
+// device gives its places up as it ends.  If the tiles have not all arrived
+// within a quarter second (another process holds the GPU, or work this library
+// does not know of), the launch ends without having changed anything and says
+// so, and the caller takes the other kernels; until then the tiles that have
+// arrived hold their places.  Waits inside the run are bounded too.
 #include "ep2d_internal.h"
 #include "ep2d_march.h"
 
@@ -49,9 +50,6 @@
 namespace ep2d {
 
 namespace {
-
-// tiles in flight on this device, in half CUs
-__device__ unsigned g_resInUse;
 
 __device__ __forceinline__ unsigned ald(unsigned* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -66,16 +64,13 @@ __device__ __forceinline__ unsigned acas(unsigned* p, unsigned from, unsigned to
 }
 
 // Arrival of one workgroup (its first thread): the state all of them see.  The
-// first to arrive decides: it reserves the room, waits for the others and
-// lets the run go, or ends it.  (The others' bound is longer: it only serves
+// first to arrive decides: it waits for the others and lets the run go, or
+// ends it.  (The others' bound is longer: it only serves
 // if the first never decides.)
-__device__ unsigned res_arrive(ResCtl* c, unsigned tiles, unsigned cost, unsigned cap,
-                               unsigned ticks) {
+__device__ unsigned res_arrive(ResCtl* c, unsigned tiles, unsigned ticks) {
   const unsigned long long t0 = wall_clock64();
   if (aadd(&c->arrive, 1u) == 0) {
-    const unsigned need = tiles * cost;
     unsigned how = ticks ? kResGo : kResLate;
-    if (aadd(&g_resInUse, need) + need > cap) how = kResNoRoom;
     while (how == kResGo && ald(&c->arrive) < tiles) {
       if (wall_clock64() - t0 > ticks) how = kResLate;
       __builtin_amdgcn_s_sleep(1);
@@ -94,18 +89,17 @@ __device__ unsigned res_arrive(ResCtl* c, unsigned tiles, unsigned cost, unsigne
   }
 }
 
-// Departure: the last workgroup gives the room back (also that of a run that
-// did not find enough), tells the host how the
-// launch went and clears the record for the next one.
-__device__ void res_depart(ResCtl* c, unsigned tiles, unsigned cost, unsigned* told) {
+// Departure: the last workgroup clears the record for the next launch and tells
+// the host how this one went.
+__device__ void res_depart(ResCtl* c, unsigned tiles, unsigned run, unsigned* told) {
   __builtin_amdgcn_s_waitcnt(0);
   if (aadd(&c->depart, 1u) + 1 != tiles) return;
   const unsigned s = ald(&c->state);
-  aadd(&g_resInUse, 0u - tiles * cost);
   __hip_atomic_store(&c->arrive, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __hip_atomic_store(&c->depart, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __hip_atomic_store(&c->state, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(told, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (s == kResGo) __hip_atomic_store(told, run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  else __hip_atomic_store(told + 1, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The exchange buffer is read and written through a buffer resource, past the
@@ -809,8 +803,8 @@ constexpr int res_waves() {
 template <typename CT, typename VT, int R, int T, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(res_waves<CT, R>()))) void k_resident(
     const RveDev* __restrict__ rves, const ResTile* __restrict__ tiles, int parity, int vpar,
-    int n, const char* xch, unsigned xpar, unsigned tag0, ResCtl* ctl, unsigned cost,
-    unsigned cap, ResLimits lim, unsigned* told) {
+    int n, const char* xch, unsigned xpar, unsigned tag0, ResCtl* ctl, ResLimits lim, unsigned run,
+    unsigned* told) {
   using Lds = ResLds<CT, VT, R, T, NW>;
   __shared__ Lds lds;
   const int v = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -824,7 +818,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(res_wav
       (&lds.zeroV[0][0][0])[2 * threadIdx.x + 1] = (VT)0;
     }
   }
-  if (threadIdx.x == 0) lds.state = res_arrive(ctl, gridDim.x, cost, cap, lim.arriveTicks);
+  if (threadIdx.x == 0) lds.state = res_arrive(ctl, gridDim.x, lim.arriveTicks);
   __syncthreads();
   if (lds.state == kResGo) {
     bool lost = false;
@@ -864,7 +858,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(res_wav
     if (__any(lost) && (threadIdx.x & 63) == 0) acas(&ctl->state, kResGo, kResLost);
   }
   __syncthreads();
-  if (threadIdx.x == 0) res_depart(ctl, gridDim.x, cost, told);
+  if (threadIdx.x == 0) res_depart(ctl, gridDim.x, run, told);
 }
 
 // the kernel of a scheme and a tile shape
@@ -946,10 +940,10 @@ int resident_tiles(const ResShape& sh, int mode, int n, int rve, size_t x0, ResT
   return t;
 }
 
-int resident_room(int device) {
+int device_cus(int device) {
   int cus = 0;
   EP2D_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-  return 2 * cus;
+  return cus;
 }
 
 int resident_cost(const ResShape& sh, int mode) {
@@ -967,10 +961,10 @@ void launch_resident(const ResLaunch& a, hipStream_t s, hipEvent_t e0, hipEvent_
     const char* xch = a.xch;
     if (e0)
       hipExtLaunchKernelGGL(kern, grid, block, 0, s, e0, e1, 0, a.rves, a.list, a.parity, a.vpar,
-                            a.iters, xch, a.xpar, a.tag0, a.ctl, a.cost, a.room, a.limits, a.told);
+                            a.iters, xch, a.xpar, a.tag0, a.ctl, a.limits, a.run, a.told);
     else
       hipLaunchKernelGGL(kern, grid, block, 0, s, a.rves, a.list, a.parity, a.vpar, a.iters, xch,
-                         a.xpar, a.tag0, a.ctl, a.cost, a.room, a.limits, a.told);
+                         a.xpar, a.tag0, a.ctl, a.limits, a.run, a.told);
     return 0;
   });
   EP2D_HIP(hipGetLastError());

@@ -1,0 +1,95 @@
+// ep2d_room.h -- which handles of this process are at work on a device, and
+// which of them may run resident (ep2d_resident.hip) side by side.
+#pragma once
+
+#include <algorithm>
+#include <map>
+#include <mutex>
+#include <vector>
+
+#include "ep2d_internal.h"
+
+namespace ep2d {
+
+// Room of resident tiles: `whole` tiles take a CU each, two `half` ones share
+// one.  Half tiles spread one to a CU while CUs are free, so beside whole tiles
+// each counts as a CU: then every tile of the launches let in finds its place,
+// in whatever order they start and end.
+inline bool resident_fits(unsigned cus, unsigned half, unsigned whole) {
+  return whole == 0 ? half <= 2 * cus : half + whole <= cus;
+}
+
+// What one handle has on a device.  Its fields are the room's while the handle
+// is in it.
+struct RoomUser {
+  hipStream_t stream = nullptr;      // its work
+  unsigned half = 0, whole = 0;      // its resident tiles (0, 0: it has no such shape)
+  const unsigned* told = nullptr;    // pinned words a resident run writes when it ends
+  unsigned run = 0;                  // the resident run it has in flight (0: none)
+  bool atWork = false;               // other work may be in flight
+  bool held = false;                 // its stream must not be asked (a capture is on)
+};
+
+// The words: the last run that has completed, and how a run failed (0: none did).
+inline bool run_ended(const unsigned* told, unsigned run) {
+  return __atomic_load_n(told, __ATOMIC_ACQUIRE) == run ||
+         __atomic_load_n(told + 1, __ATOMIC_ACQUIRE) != 0;
+}
+
+// The handles of this process on one device.
+class DeviceRoom {
+ public:
+  static DeviceRoom& of(int device) {
+    // never destroyed: handles may outlive static objects
+    static std::mutex* m = new std::mutex;
+    static auto* rooms = new std::map<int, DeviceRoom>;
+    const std::lock_guard<std::mutex> lock(*m);
+    return (*rooms)[device];
+  }
+  void join(RoomUser* u) {
+    const std::lock_guard<std::mutex> lock(m_);
+    users_.push_back(u);
+  }
+  // (its work is done: the stream is idle)
+  void leave(RoomUser* u) {
+    const std::lock_guard<std::mutex> lock(m_);
+    users_.erase(std::remove(users_.begin(), users_.end(), u), users_.end());
+  }
+  // Before work of `me` is enqueued.  With run != 0: whether that resident run may
+  // be launched, which it may if all handles at work fit the device with their
+  // resident tiles (one that has no such shape leaves no room).
+  bool enter(RoomUser* me, unsigned run, unsigned cus) {
+    const std::lock_guard<std::mutex> lock(m_);
+    unsigned half = me->half, whole = me->whole;
+    bool all = run != 0;
+    for (RoomUser* u : users_) {
+      if (!all) break;
+      if (u == me || !busy(*u)) continue;
+      half += u->half;
+      whole += u->whole;
+      all = u->half + u->whole > 0 && resident_fits(cus, half, whole);
+    }
+    all = all && resident_fits(cus, half, whole);
+    me->run = all ? run : 0;
+    me->atWork = !all;
+    return all;
+  }
+  void hold(RoomUser* me, bool on) {
+    const std::lock_guard<std::mutex> lock(m_);
+    me->held = on;
+  }
+
+ private:
+  static bool busy(RoomUser& u) {
+    if (u.run != 0 && run_ended(u.told, u.run)) u.run = 0;
+    if (u.atWork && !u.held) {
+      if (hipStreamQuery(u.stream) == hipSuccess) u.atWork = false;
+      else (void)hipGetLastError();
+    }
+    return u.run != 0 || u.atWork;
+  }
+  std::mutex m_;
+  std::vector<RoomUser*> users_;
+};
+
+}  // namespace ep2d

@@ -185,6 +185,7 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
   EP2D_HIP(hipGetDeviceCount(&ndev));
   if (device_ < 0 || device_ >= ndev) throw ArgError("device index out of range");
   EP2D_HIP(hipSetDevice(device_));
+  cus_ = (unsigned)device_cus(device_);
   if (stream) {
     stream_ = stream;
     ownStream_ = false;
@@ -408,6 +409,11 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
     }
   }
   EP2D_HIP(hipStreamSynchronize(stream_));
+  if (ownStream_) {
+    room_.stream = stream_;
+    inRoom_ = &DeviceRoom::of(device_);
+    inRoom_->join(&room_);
+  }
 
   if (!logPath_.empty()) log_.open(logPath_, std::ios_base::app);   // :1607
 }
@@ -415,19 +421,22 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
 // Shape of the resident runs of a handle on the automatic shape, and its tiles.
 void Solver::planResident(std::vector<ResTile>& tiles) {
   if (nX_ < kResMinSide) return;
-  resRoom_ = (unsigned)resident_room(device_);
   for (const ResShape& sh : resident_shapes(mode_)) {
     size_t pairs = 0;
     const int n = resident_tiles(sh, mode_, nX_, 0, 0, nullptr, &pairs);
     const int cost = n > 0 ? resident_cost(sh, mode_) : 0;
-    if (cost == 0 || (size_t)n * (size_t)cost > resRoom_ || pairs * 16 > 0x7fffffffu) continue;
+    const unsigned half = cost == 1 ? (unsigned)n : 0, whole = cost == 1 ? 0 : (unsigned)n;
+    if (cost == 0 || !resident_fits(cus_, half, whole) || pairs * 16 > 0x7fffffffu) continue;
     tiles.resize((size_t)n);
     resident_tiles(sh, mode_, nX_, 0, 0, tiles.data(), nullptr);
     resShape_ = sh;
-    resCost_ = (unsigned)cost;
+    room_.half = half;
+    room_.whole = whole;
     resXpar_ = (unsigned)((pairs * 16 + 255) / 256 * 256);
     resTiles_ = n;
-    hResTold_ = (unsigned*)(hMax_ + 3);  // the word past the residual's three
+    hResTold_ = (unsigned*)(hMax_ + 3);  // the words past the residual's three
+    hResTold_[0] = hResTold_[1] = 0;
+    room_.told = hResTold_;
     lastResident_ = true;
     return;
   }
@@ -435,14 +444,20 @@ void Solver::planResident(std::vector<ResTile>& tiles) {
 
 // Whether n iterations run resident now: a handle with such a shape, and enough
 // iterations to pay for the start (the tiles' arrival and the loads of the
-// state take about ten microseconds).
+// state take about ten microseconds), and room beside the other handles at work.
 bool Solver::residentFits(long n) {
   if (resTiles_ == 0 || n < kResMinIters || stress64_) return false;
   if (resSkip_ > 0) {
     resSkip_--;
     return false;
   }
-  return true;
+  if (++resRun_ == 0) resRun_ = 1;
+  return inRoom_->enter(&room_, resRun_, cus_);
+}
+
+// Before launches of the other kernels: the handle is at work.
+void Solver::enterRoom() {
+  if (inRoom_) inRoom_->enter(&room_, 0, cus_);
 }
 
 void Solver::launchResidentRun(long n) {
@@ -466,11 +481,9 @@ void Solver::launchResidentRun(long n) {
   a.xpar = resXpar_;
   a.tag0 = resTag_;
   a.ctl = dResCtl_;
-  a.cost = resCost_;
-  a.room = resRoom_;
   a.limits = resLimits_;
+  a.run = resRun_;
   a.told = hResTold_;
-  *hResTold_ = 0;
   launch_resident(a, stream_, timed ? ev.first : nullptr, timed ? ev.second : nullptr);
   resTag_ += (unsigned)n;
   resPending_ = n;
@@ -489,23 +502,25 @@ bool Solver::settled() {
   if (resPending_ == 0) return true;
   const long n = resPending_;
   resPending_ = 0;
-  const unsigned how = *hResTold_;
-  if (how == kResGo) {
+  const unsigned how = hResTold_[1];
+  if (how == 0) {
     resCounts_[0]++;
     return true;
   }
+  hResTold_[1] = 0;
   // the launch computed nothing: its duration is no sample
   if (!pending_.empty() && pending_.back().kind == kTimedResident) {
     freeEvents_.push_back(pending_.back().ev);
     pending_.pop_back();
   }
-  const bool lost = how != kResNoRoom && how != kResLate;
+  const bool lost = how != kResLate;
   resCounts_[lost ? 2 : 1]++;
-  if (lost || how == kResLate) resSkip_ = 256;
+  resSkip_ = 256;
   if (lost) {
     // U and V are torn: no call uses them until they are set again (the
     // stress fields are as in a new handle)
     lostFields_ = 15;
+    enterRoom();
     const size_t nC = (size_t)nX_ * nY_, nV = (size_t)(nX_ - 1) * (nY_ - 1);
     for (double* p : {f_.P, f_.tauXX, f_.tauYY, f_.tauXYav, f_.J2})
       launch_fill(p, nC, 0.0, stream_);
@@ -562,6 +577,8 @@ void Solver::release() {
   // teardown: errors are ignored, there is no caller to report them to
   (void)hipSetDevice(device_);
   if (stream_) (void)hipStreamSynchronize(stream_);
+  if (inRoom_) inRoom_->leave(&room_);
+  inRoom_ = nullptr;
   dropPlainGraph();
   for (auto& p : pending_) freeEvents_.push_back(p.ev);
   for (auto& e : freeEvents_) {
@@ -819,16 +836,23 @@ long Solver::replayPlain(long n) {
   if (!plainExec_) {
     std::memcpy(&plainRve_, &r_, sizeof(r_));
     const long launches = launchCount_;
-    EP2D_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
-    try {
-      for (long k = 0; k < kPlainGraph; k++) launchIteration();
-    } catch (...) {
-      hipGraph_t g = nullptr;
-      (void)hipStreamEndCapture(stream_, &g);
-      if (g) (void)hipGraphDestroy(g);
-      throw;
+    // (another thread's question to a stream that captures would end the capture)
+    inRoom_->hold(&room_, true);
+    hipError_t ended = hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal);
+    if (ended == hipSuccess) {
+      try {
+        for (long k = 0; k < kPlainGraph; k++) launchIteration();
+      } catch (...) {
+        hipGraph_t g = nullptr;
+        (void)hipStreamEndCapture(stream_, &g);
+        if (g) (void)hipGraphDestroy(g);
+        inRoom_->hold(&room_, false);
+        throw;
+      }
+      ended = hipStreamEndCapture(stream_, &plainGraph_);
     }
-    EP2D_HIP(hipStreamEndCapture(stream_, &plainGraph_));
+    inRoom_->hold(&room_, false);
+    EP2D_HIP(ended);
     EP2D_HIP(hipGraphInstantiate(&plainExec_, plainGraph_, nullptr, nullptr, 0));
     launchCount_ = launches;
   }
@@ -846,7 +870,10 @@ void Solver::dropPlainGraph() {
 }
 
 void Solver::iterateLaunches(long n) {
-  if (n > 0) lastResident_ = false;
+  if (n > 0) {
+    lastResident_ = false;
+    enterRoom();
+  }
   n -= replayPlain(n);
   if (!multiIter_ || (stress64_ && !multi64())) {
     for (long k = 0; k < n; k++) launchIteration();

@@ -9,6 +9,7 @@
 
 #include "../../include/ep2d.h"
 #include "ep2d_internal.h"
+#include "ep2d_room.h"
 
 namespace ep2d {
 
@@ -192,7 +193,9 @@ class Solver {
   // the run whose outcome has not been read yet (its iterations, 0: none)
   int resTiles_ = 0;
   ResShape resShape_;
-  unsigned resCost_ = 0, resRoom_ = 0, resTag_ = 0, resXpar_ = 0;
+  unsigned resRun_ = 0, resTag_ = 0, resXpar_ = 0, cus_ = 0;
+  RoomUser room_;                   // this handle among those on the device
+  DeviceRoom* inRoom_ = nullptr;    // (null: on a caller's stream, or its engine's)
   ResTile* dResTiles_ = nullptr;
   char* dXch_ = nullptr;
   ResCtl* dResCtl_ = nullptr;
@@ -203,6 +206,7 @@ class Solver {
   int resSkip_ = 0;                 // runs to take the other kernels after a late start
   void planResident(std::vector<ResTile>& tiles);
   bool residentFits(long n);
+  void enterRoom();
   void launchResidentRun(long n);
   bool settled();                   // after the stream is synchronised
   void settleRun();

@@ -293,7 +293,7 @@ int ep2d_diag_chain_order(const int* segs, int n, int stageWaves, const int* dim
 /* Diagnostic, no counterpart in the reference: the resident runs of a handle
  * (runs of 16 iterations and more of a grid that fits on the chip, in one
  * launch).  counts (3 words, may be NULL) receives the runs completed, those
- * whose workgroups could not all start (their iterations took the other
+ * whose workgroups did not all start in time (their iterations took the other
  * kernels: the same results) and those that lost a wait inside the run.
  * After a lost one (reported once as EP2D_ERR_HIP) the calls that use the state
  * return EP2D_ERR_STATE until Ux, Uy, Vx and Vy have been set.

@@ -3,6 +3,9 @@ runs are counted by their outcome, so a run that was meant to be resident is
 seen to be one, and the paths a busy device takes are forced from the host (a
 launch that may not wait for its workgroups).  Every path gives the tile
 kernel's bits (no tolerance)."""
+import threading
+import time
+
 import numpy as np
 import pytest
 # torch before the library: one HIP runtime in the process
@@ -198,3 +201,71 @@ def test_one_late_start_a_call():
         a = {k: g.get(k) for k in FIELDS}
         assert g.diag_resident() == (0, 1, 0)
     _same(a, _tiles(nX, "split", pa, init, n))
+
+
+def test_room_beside_another_run():
+    """Tiles of half a CU each may lie one to a CU: beside a run of 252 of them 16
+    more half tiles run resident, a grid of 48 whole-CU tiles (on 256 CUs) takes
+    the chains at once and does not wait for that run."""
+    print("room", flush=True)
+    cases = [("split", 333, 60000), ("split", 64, 500), ("fp64", 128, 500)]
+    hs, inits = [], []
+    try:
+        for mode, nX, _ in cases:
+            pa, init = _case(nX, mode, 2 + nX)
+            hs.append(EffPlast2D(pa, nX, nTasks=3, mode=mode))
+            inits.append((pa, init))
+            _start(hs[-1], init)
+        for h in hs:        # (the first launches of the kernels load them)
+            h.iterate(20)
+            h.sync()
+        t0 = time.perf_counter()
+        ends = []
+        for h, (_, _, n) in zip(hs, cases):
+            h.iterate(n)
+        for h in hs[1:] + hs[:1]:
+            h.sync()
+            ends.append(time.perf_counter() - t0)
+        print("ends", ends, flush=True)
+        assert [h.diag_resident() for h in hs] == [(2, 0, 0), (2, 0, 0), (1, 0, 0)]
+        assert max(ends[:2]) < 0.5 * ends[2]
+        for h, (mode, nX, n), (pa, init) in zip(hs, cases, inits):
+            if n < 1000:
+                _same({k: h.get(k) for k in FIELDS}, _tiles(nX, mode, pa, init, n + 20))
+    finally:
+        for h in hs:
+            h.close()
+
+
+def test_plain_capture_beside_other_handles():
+    """Plain handles capture their runs on one thread while another thread's handle
+    asks which handles are at work."""
+    print("plain capture beside another thread", flush=True)
+    nX, n = 33, 250
+    pa, init = _case(nX, "plain", 1)
+    errors = []
+
+    def plain():
+        try:
+            with EffPlast2D(pa, nX, nTasks=3, mode="plain", tileRows=0) as g:
+                _start(g, init)
+                for _ in range(10):
+                    g.iterate(25)
+                ref = {k: g.get(k) for k in FIELDS}
+            for _ in range(20):
+                with EffPlast2D(pa, nX, nTasks=3, mode="plain") as g:
+                    _start(g, init)
+                    g.iterate(n)
+                    _same({k: g.get(k) for k in FIELDS}, ref)
+        except Exception as e:      # noqa: BLE001
+            errors.append(e)
+
+    th = threading.Thread(target=plain)
+    with EffPlast2D(pa, nX, nTasks=3, mode="fp64") as g:
+        _start(g, init)
+        th.start()
+        while th.is_alive():
+            g.iterate(16)
+            g.sync()
+        th.join()
+    assert not errors, errors
