@@ -197,10 +197,11 @@ struct ResTile {
   int xl, xr, xu, xd;
   int pad;
 };
-// Arrivals and departures of a launch's workgroups and how it went; zero
-// between launches.
+// Arrivals and departures of a launch's workgroups and how it went, zero between
+// launches; failed: a launch did not run, so those after it do not either until
+// the host has cleared this.
 struct ResCtl {
-  unsigned arrive, state, depart, pad;
+  unsigned arrive, state, depart, failed;
 };
 // Bounds of a launch's waits: for its other tiles (ticks of 10 ns; 0: it does not
 // start) and for the words of one exchange (polls of about a
@@ -210,8 +211,8 @@ struct ResLimits {
 };
 // how a launch went: run, or ended with the fields untouched because its tiles
 // did not all start in time; lost: a wait inside the run ended at its bound
-// (the fields are not valid)
-constexpr unsigned kResGo = 1, kResLate = 2, kResLost = 3;
+// (the fields are not valid); after: an earlier launch did not run
+constexpr unsigned kResGo = 1, kResLate = 2, kResLost = 3, kResAfter = 4;
 constexpr long kResMinIters = 16;  // shorter runs take the other kernels
 constexpr int kResMinSide = 16;
 struct ResLaunch {

@@ -40,8 +40,9 @@
 // device gives its places up as it ends.  If the tiles have not all arrived
 // within a quarter second (another process holds the GPU, or work this library
 // does not know of), the launch ends without having changed anything and says
-// so, and the caller takes the other kernels; until then the tiles that have
-// arrived hold their places.  Waits inside the run are bounded too.
+// so, those queued behind it do the same, and the caller takes the other kernels;
+// until then the tiles that have arrived hold their places.  Waits inside the
+// run are bounded too.
 #include "ep2d_internal.h"
 #include "ep2d_march.h"
 
@@ -70,7 +71,7 @@ __device__ __forceinline__ unsigned acas(unsigned* p, unsigned from, unsigned to
 __device__ unsigned res_arrive(ResCtl* c, unsigned tiles, unsigned ticks) {
   const unsigned long long t0 = wall_clock64();
   if (aadd(&c->arrive, 1u) == 0) {
-    unsigned how = ticks ? kResGo : kResLate;
+    unsigned how = ald(&c->failed) != 0u ? kResAfter : ticks ? kResGo : kResLate;
     while (how == kResGo && ald(&c->arrive) < tiles) {
       if (wall_clock64() - t0 > ticks) how = kResLate;
       __builtin_amdgcn_s_sleep(1);
@@ -98,8 +99,12 @@ __device__ void res_depart(ResCtl* c, unsigned tiles, unsigned run, unsigned* to
   __hip_atomic_store(&c->arrive, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __hip_atomic_store(&c->depart, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __hip_atomic_store(&c->state, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (s == kResGo) __hip_atomic_store(told, run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  else __hip_atomic_store(told + 1, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (s == kResGo) {
+    __hip_atomic_store(told, run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  } else if (s != kResAfter) {
+    __hip_atomic_store(&c->failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(told + 1, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 // The exchange buffer is read and written through a buffer resource, past the

@@ -56,10 +56,15 @@ class DeviceRoom {
     users_.erase(std::remove(users_.begin(), users_.end(), u), users_.end());
   }
   // Before work of `me` is enqueued.  With run != 0: whether that resident run may
-  // be launched, which it may if all handles at work fit the device with their
-  // resident tiles (one that has no such shape leaves no room).
+  // be launched, which it may behind a run of `me` still in flight, or if all
+  // handles at work fit the device with their resident tiles (one that has no
+  // such shape leaves no room).
   bool enter(RoomUser* me, unsigned run, unsigned cus) {
     const std::lock_guard<std::mutex> lock(m_);
+    if (run != 0 && me->run != 0 && !run_ended(me->told, me->run)) {
+      me->run = run;
+      return true;
+    }
     unsigned half = me->half, whole = me->whole;
     bool all = run != 0;
     for (RoomUser* u : users_) {

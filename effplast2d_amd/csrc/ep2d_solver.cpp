@@ -447,6 +447,8 @@ void Solver::planResident(std::vector<ResTile>& tiles) {
 // state take about ten microseconds), and room beside the other handles at work.
 bool Solver::residentFits(long n) {
   if (resTiles_ == 0 || n < kResMinIters || stress64_) return false;
+  noteRuns();
+  if (__atomic_load_n(hResTold_ + 1, __ATOMIC_ACQUIRE) != 0) settle();
   if (resSkip_ > 0) {
     resSkip_--;
     return false;
@@ -486,32 +488,45 @@ void Solver::launchResidentRun(long n) {
   a.told = hResTold_;
   launch_resident(a, stream_, timed ? ev.first : nullptr, timed ? ev.second : nullptr);
   resTag_ += (unsigned)n;
-  resPending_ = n;
+  resRuns_.push_back({resRun_, n});
   cur_ ^= 1;
   stressStale_ = true;
-  // (the newest samples stay unread until the run's outcome is known)
-  if (timed) noteTimed(ev, kTimedResident, n);
+  if (timed) noteTimed(ev, kTimedResident, n, resRun_);
   launchCount_++;
   lastResident_ = true;
 }
 
-// Outcome of the last resident run, the stream being idle: true when there
-// was none or it ran; else its iterations have been launched on the other
-// kernels.
-bool Solver::settled() {
-  if (resPending_ == 0) return true;
-  const long n = resPending_;
-  resPending_ = 0;
-  const unsigned how = hResTold_[1];
-  if (how == 0) {
+void Solver::noteRuns() {
+  const unsigned done = __atomic_load_n(hResTold_, __ATOMIC_ACQUIRE);
+  while (!resRuns_.empty() && (int)(done - resRuns_.front().run) >= 0) {
+    resRuns_.pop_front();
     resCounts_[0]++;
-    return true;
   }
+}
+
+// Outcome of the resident runs, the stream being idle: true when there was none
+// or they ran; else their iterations, from the first that did not run, have
+// been launched on the other kernels.
+bool Solver::settled() {
+  if (resRuns_.empty()) return true;
+  noteRuns();
+  const unsigned how = hResTold_[1];
+  if (how == 0 && resRuns_.empty()) return true;
+  long n = 0;
+  for (const ResRun& q : resRuns_) n += q.iters;
+  if (resRuns_.size() & 1) cur_ ^= 1;
+  resRuns_.clear();
+  launch_fill((double*)dResCtl_, sizeof(ResCtl) / 8, 0.0, stream_);
   hResTold_[1] = 0;
-  // the launch computed nothing: its duration is no sample
-  if (!pending_.empty() && pending_.back().kind == kTimedResident) {
-    freeEvents_.push_back(pending_.back().ev);
-    pending_.pop_back();
+  // these launches computed nothing: their durations are no samples
+  const unsigned done = hResTold_[0];
+  for (size_t k = 0; k < pending_.size();) {
+    if (pending_[k].kind == kTimedResident && (int)(pending_[k].run - done) > 0) {
+      freeEvents_.push_back(pending_[k].ev);
+      pending_.erase(pending_.begin() + (long)k);
+    } else {
+      k++;
+    }
   }
   const bool lost = how != kResLate;
   resCounts_[lost ? 2 : 1]++;
@@ -528,14 +543,14 @@ bool Solver::settled() {
     stressStale_ = false;
     throw HipError("a resident run lost a wait for a neighbouring tile");
   }
-  cur_ ^= 1;
   iterateLaunches(n);
   return false;
 }
 
-// A resident run's outcome is known.
+// The resident runs' outcome is known.
 void Solver::settleRun() {
-  if (resPending_ == 0) return;
+  if (!resRuns_.empty()) noteRuns();
+  if (resRuns_.empty()) return;
   EP2D_HIP(hipSetDevice(device_));
   EP2D_HIP(hipStreamSynchronize(stream_));
   settled();
@@ -759,8 +774,9 @@ std::pair<hipEvent_t, hipEvent_t> Solver::takeTimingEvents() {
   return ev;
 }
 
-void Solver::noteTimed(const std::pair<hipEvent_t, hipEvent_t>& ev, TimedKind kind, long iters) {
-  pending_.push_back({ev, kind, iters});
+void Solver::noteTimed(const std::pair<hipEvent_t, hipEvent_t>& ev, TimedKind kind, long iters,
+                       unsigned run) {
+  pending_.push_back({ev, kind, iters, run});
   if (pending_.size() >= 256) resolveTiming(false);
 }
 
@@ -806,17 +822,18 @@ int Solver::iterMode() const { return stress64_ ? kModeSplitStress64 : mode_; }
 
 void Solver::iterate(long n) {
   EP2D_HIP(hipSetDevice(device_));
-  settle();
-  // (a launch of a second at most, which other handles' work may wait for; what
-  // follows one that started late takes the other kernels)
+  requireState();
+  // resident runs queue up behind each other (launches of a second at most,
+  // which other handles' work may wait for); the other kernels' launches wait
+  // until their outcome is known
   constexpr long kMost = 1L << 16;
   while (residentFits(n)) {
     const long m = std::min(n, kMost);
     launchResidentRun(m);
     n -= m;
     if (n == 0) return;
-    settle();
   }
+  settle();
   iterateLaunches(n);
 }
 
@@ -922,6 +939,10 @@ void Solver::resolveTiming(bool all) {
     pending_.erase(pending_.begin());
     freeEvents_.push_back(p.ev);
     EP2D_HIP(hipEventSynchronize(p.ev.second));
+    // (a resident launch that did not run computed nothing)
+    if (p.kind == kTimedResident &&
+        (int)(p.run - __atomic_load_n(hResTold_, __ATOMIC_ACQUIRE)) > 0)
+      continue;
     float ms = 0.f;
     EP2D_HIP(hipEventElapsedTime(&ms, p.ev.first, p.ev.second));
     timedMs_ += ms;          // averages are per iteration

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <chrono>
+#include <deque>
 #include <fstream>
 #include <string>
 #include <unordered_map>
@@ -190,7 +191,7 @@ class Solver {
   void flipV();                     // the other velocity buffer becomes current
   // resident runs (ep2d_resident.hip): the shape of this grid (resTiles_ 0:
   // none), its tile list, exchange buffer and launch record in one block, and
-  // the run whose outcome has not been read yet (its iterations, 0: none)
+  // the runs whose outcome has not been read yet, in their order
   int resTiles_ = 0;
   ResShape resShape_;
   unsigned resRun_ = 0, resTag_ = 0, resXpar_ = 0, cus_ = 0;
@@ -200,7 +201,11 @@ class Solver {
   char* dXch_ = nullptr;
   ResCtl* dResCtl_ = nullptr;
   unsigned* hResTold_ = nullptr;
-  long resPending_ = 0;
+  struct ResRun {
+    unsigned run;
+    long iters;
+  };
+  std::deque<ResRun> resRuns_;
   ResLimits resLimits_;
   long long resCounts_[3] = {0, 0, 0};  // completed, turned away or late, lost
   int resSkip_ = 0;                 // runs to take the other kernels after a late start
@@ -208,6 +213,7 @@ class Solver {
   bool residentFits(long n);
   void enterRoom();
   void launchResidentRun(long n);
+  void noteRuns();                  // drop the runs known to have completed
   bool settled();                   // after the stream is synchronised
   void settleRun();
   void settle();
@@ -260,6 +266,7 @@ class Solver {
     std::pair<hipEvent_t, hipEvent_t> ev;
     TimedKind kind;
     long iters;
+    unsigned run;  // resident: its number
   };
   std::vector<TimedLaunch> pending_;   // sampled launches not read yet
   std::vector<std::pair<hipEvent_t, hipEvent_t>> freeEvents_;
@@ -268,7 +275,8 @@ class Solver {
   long timedOf_[kTimedKinds] = {0};  // the samples by kernel
   bool lastResident_ = false;        // the last iterations ran resident
   std::pair<hipEvent_t, hipEvent_t> takeTimingEvents();
-  void noteTimed(const std::pair<hipEvent_t, hipEvent_t>& ev, TimedKind kind, long iters);
+  void noteTimed(const std::pair<hipEvent_t, hipEvent_t>& ev, TimedKind kind, long iters,
+                 unsigned run = 0);
   std::string kernelName(TimedKind kind) const;
   std::string timingName_;         // kernel name getTiming() hands out
 

@@ -235,7 +235,10 @@ int ep2d_field_device(ep2d_handle* h, int field, const void** ptr);
 int ep2d_get_mask(ep2d_handle* h, unsigned char* host, size_t count);
 
 /* ---- step-level entry points (the pieces ComputeEffParams is made of) ----*/
-/* n iterations of the handle's scheme, no residual checks (:389-399). */
+/* n iterations of the handle's scheme, no residual checks (:389-399).  The work
+ * is queued; on a handle with its own stream, a call of fewer than 16
+ * iterations (and ep2d_apply_affine) behind a resident run waits for it
+ * (ep2d_diag_resident). */
 int ep2d_iterate(ep2d_handle* h, long n);
 /* U += affine field of the macro strain increment (:370-381), on device. */
 int ep2d_apply_affine(ep2d_handle* h, double dUxdx, double dUydy,

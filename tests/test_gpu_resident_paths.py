@@ -269,3 +269,41 @@ def test_plain_capture_beside_other_handles():
             g.sync()
         th.join()
     assert not errors, errors
+
+
+@pytest.mark.parametrize("mode", ["fp64", "split"])
+def test_runs_queue_up(mode):
+    """Resident runs are queued behind each other: the calls return at once, and
+    a launch that did not start keeps those behind it from running."""
+    nX = 125
+    print(f"queued runs {mode}", flush=True)
+    pa, init = _case(nX, mode, 31)
+    with EffPlast2D(pa, nX, nTasks=3, mode=mode) as g:
+        _start(g, init)
+        g.iterate(16)
+        g.sync()
+        t0 = time.perf_counter()
+        for n in (20001, 30, 16, 20000):
+            g.iterate(n)
+        t1 = time.perf_counter()
+        g.sync()
+        t2 = time.perf_counter()
+        assert t1 - t0 < 0.25 * (t2 - t0)
+        a = {k: g.get(k) for k in FIELDS}
+        assert g.diag_resident() == (5, 0, 0)
+        _same(a, _tiles(nX, mode, pa, init, 40063))
+        # two run, the third does not start, nor the two queued behind it
+        _start(g, init)
+        g.iterate(3000)
+        g.iterate(17)
+        g.diag_resident(arrive_ticks=0)
+        g.set_timing(1)
+        for n in (18, 16, 19):
+            g.iterate(n)
+        ms, samples, name = g.timing()
+        a = {k: g.get(k) for k in FIELDS}
+        done, late, lost = g.diag_resident()
+        assert (done, lost) == (7, 0) and late >= 1
+        # (16-step launches of four, one on its own: closing ones are no samples)
+        assert "k_chain" in name and samples <= 53
+        _same(a, _tiles(nX, mode, pa, init, 3000 + 17 + 53))
