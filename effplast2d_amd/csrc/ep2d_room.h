@@ -55,29 +55,35 @@ class DeviceRoom {
     const std::lock_guard<std::mutex> lock(m_);
     users_.erase(std::remove(users_.begin(), users_.end(), u), users_.end());
   }
-  // Before work of `me` is enqueued.  With run != 0: whether that resident run may
-  // be launched, which it may behind a run of `me` still in flight, or if all
-  // handles at work fit the device with their resident tiles (one that has no
-  // such shape leaves no room).
-  bool enter(RoomUser* me, unsigned run, unsigned cus) {
+  // Before work of `me` is enqueued: 0 if the resident run `run` (0: none) may be
+  // launched, else the handles at work, `me` among them (counted to 3).  It may
+  // be if all handles at work fit the device with their resident tiles (one
+  // that has no such shape leaves no room).
+  int enter(RoomUser* me, unsigned run, unsigned cus) {
     const std::lock_guard<std::mutex> lock(m_);
-    if (run != 0 && me->run != 0 && !run_ended(me->told, me->run)) {
-      me->run = run;
-      return true;
-    }
     unsigned half = me->half, whole = me->whole;
+    int n = 1;
     bool all = run != 0;
     for (RoomUser* u : users_) {
-      if (!all) break;
+      if (!all && n >= 3) break;
       if (u == me || !busy(*u)) continue;
+      n++;
       half += u->half;
       whole += u->whole;
-      all = u->half + u->whole > 0 && resident_fits(cus, half, whole);
+      all = all && u->half + u->whole > 0;
     }
     all = all && resident_fits(cus, half, whole);
-    me->run = all ? run : 0;
-    me->atWork = !all;
-    return all;
+    // (a run that is turned down leaves those before it in the entry; the other
+    // kernels' launches, run 0, come when the handle has none in flight)
+    if (all || run == 0) me->run = run;
+    if (run == 0) me->atWork = true;
+    return all ? 0 : n;
+  }
+  // Before launches that do not depend on the others'.
+  void work(RoomUser* me) {
+    const std::lock_guard<std::mutex> lock(m_);
+    me->run = 0;
+    me->atWork = true;
   }
   void hold(RoomUser* me, bool on) {
     const std::lock_guard<std::mutex> lock(m_);

@@ -28,6 +28,15 @@ double std_max(double a, double b) { return (a < b) ? b : a; }  // std::max sema
 int default_tile_rows(int mode, int nX) {
   return mode == EP2D_MODE_FP64 && nX >= 1024 ? 14 : 8;
 }
+
+// Rows of the shortest segments of four-stage chains on two waves whose
+// workgroups fit `places` together.
+int chain_rows(int nX, int nY, int places) {
+  const int cols = chain_cols(4, 2);
+  const int strips = (nX + cols - 1) / cols;
+  const int bands = std::max(1, places / strips);
+  return std::max(2, (nY + bands - 1) / bands);
+}
 }  // namespace
 
 // get_sigma_2D.m:3-32 (MATLAB evaluates left to right).
@@ -301,12 +310,7 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
                         !(mode_ == EP2D_MODE_FP64 && opt_.laneColumns == 2);
     if (chains) {
       int rows = n <= 2048 ? 48 : 96;
-      if (n <= 1024) {
-        const int cols = chain_cols(4, 2);
-        const int strips = (nX + cols - 1) / cols;
-        const int bands = std::max(1, chain_resident(4, 2, mode_ == EP2D_MODE_SPLIT) / strips);
-        rows = std::max(2, (nY + bands - 1) / bands);
-      }
+      if (n <= 1024) rows = chain_rows(nX, nY, chain_resident(4, 2, mode_ == EP2D_MODE_SPLIT));
       opt_.marchRows = rows;
       opt_.itersPerLaunch = 4;
       if (opt_.laneColumns != 2 && opt_.stageWaves == 0) opt_.stageWaves = 2;
@@ -339,71 +343,86 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
       // on the device (the kernel reads the current buffer as parity ^ cur)
       marchRows_ = opt_.marchRows;
       nSegs_ = march_segments(nX, nY, marchRows_, 0, nullptr);
-      std::vector<int4> segs((size_t)nSegs_), s2, c3, c2;
+      std::vector<int4> segs((size_t)nSegs_), s2[kLoads], c3[kLoads], c2[kLoads];
       march_segments(nX, nY, marchRows_, 0, segs.data());
       const int2 dims = make_int2(nX, nY);
       const bool f32 = mode_ == EP2D_MODE_SPLIT;
-      if (multiIter_) {
+      const bool ordered = multiIter_ && ipl_ >= 3 && !wide_;
+      const int res = ordered ? chain_resident(ipl_, stageWaves_, f32) : 0;
+      const int loads = tileSingles_ ? kLoads : 1;
+      for (int q = 0; q < loads && multiIter_; q++) {
+        // the heights for one, two, and three handles and more at work: segments
+        // that fill the device alone do little else than halo rows for several
+        // (us per handle iteration of 8 FP64 handles: 256^2 3.8 on 2 rows, 2.3 on
+        // the 5 of this rule, 2.5 on the tile kernel; 512^2 7 on 4 rows, 3.1 on
+        // the 16 of this rule, 4.1 on the tile kernel)
+        const int rows = q == 0 ? marchRows_ : chain_rows(nX, nY, res / (q + 1));
+        segsFor_[q].rows = rows;
         auto segsOf = [&](int4* out) {
-          if (ipl_ == 2) return march2_segments(nX, nY, marchRows_, 0, out);
-          if (wide_) return wide_segments(ipl_, nX, nY, marchRows_, 0, out);
-          return chain_segments(ipl_, nX, nY, marchRows_, 0, out, stageWaves_);
+          if (ipl_ == 2) return march2_segments(nX, nY, rows, 0, out);
+          if (wide_) return wide_segments(ipl_, nX, nY, rows, 0, out);
+          return chain_segments(ipl_, nX, nY, rows, 0, out, stageWaves_);
         };
         const int raw = segsOf(nullptr);
-        const bool ordered = ipl_ >= 3 && !wide_;
-        const int res = ordered ? chain_resident(ipl_, stageWaves_, f32) : 0;
-        s2.resize((size_t)(ordered ? chain_work_order(nullptr, raw, stageWaves_, &dims, res, nullptr)
-                                   : raw));
-        segsOf(s2.data());
-        if (ordered) chain_work_order(s2.data(), raw, stageWaves_, &dims, res, s2.data());
-      }
-      if (ipl_ >= 3) {
+        s2[q].resize((size_t)(ordered ? chain_work_order(nullptr, raw, stageWaves_, &dims, res,
+                                                         nullptr)
+                                      : raw));
+        segsOf(s2[q].data());
+        if (ordered) chain_work_order(s2[q].data(), raw, stageWaves_, &dims, res, s2[q].data());
+        if (ipl_ < 3) continue;
         // closing launches of 26 and 42 rows, of fewer on a small grid
-        const int r2 = tileSingles_ ? std::min(26, marchRows_) : 26;
-        const int r3 = tileSingles_ ? std::min(42, marchRows_) : 42;
-        c2.resize((size_t)march2_segments(nX, nY, r2, 0, nullptr));
-        march2_segments(nX, nY, r2, 0, c2.data());
+        const int r2 = tileSingles_ ? std::min(26, rows) : 26;
+        const int r3 = tileSingles_ ? std::min(42, rows) : 42;
+        c2[q].resize((size_t)march2_segments(nX, nY, r2, 0, nullptr));
+        march2_segments(nX, nY, r2, 0, c2[q].data());
         if (ipl_ == 4) {
-          const int raw = chain_segments(3, nX, nY, r3, 0, nullptr, 1);
-          const int res = chain_resident(3, 1, f32);
-          c3.resize((size_t)chain_work_order(nullptr, raw, 1, &dims, res, nullptr));
-          chain_segments(3, nX, nY, r3, 0, c3.data(), 1);
-          chain_work_order(c3.data(), raw, 1, &dims, res, c3.data());
+          const int raw3 = chain_segments(3, nX, nY, r3, 0, nullptr, 1);
+          const int res3 = chain_resident(3, 1, f32);
+          c3[q].resize((size_t)chain_work_order(nullptr, raw3, 1, &dims, res3, nullptr));
+          chain_segments(3, nX, nY, r3, 0, c3[q].data(), 1);
+          chain_work_order(c3[q].data(), raw3, 1, &dims, res3, c3[q].data());
         }
       }
-      nSegs2_ = (int)s2.size();
-      nSegsC3_ = (int)c3.size();
-      nSegsC2_ = (int)c2.size();
       std::vector<ResTile> tiles;
       if (autoShape && !pool_) planResident(tiles);
       // every table in one block, with one copy
       RveDev rd = r_;
       rd.cur = 0;
-      const std::pair<const void*, size_t> parts[] = {
-          {&rd, sizeof(rd)},
-          {segs.data(), segs.size() * sizeof(int4)},
-          {s2.data(), s2.size() * sizeof(int4)},
-          {c3.data(), c3.size() * sizeof(int4)},
-          {c2.data(), c2.size() * sizeof(int4)},
-          {tiles.data(), tiles.size() * sizeof(ResTile)}};
-      size_t at[7] = {0};
-      for (int k = 0; k < 6; k++) at[k + 1] = at[k] + (parts[k].second + 255) / 256 * 256;
-      std::vector<char> host(at[6], 0);
-      for (int k = 0; k < 6; k++)
-        if (parts[k].second) std::memcpy(host.data() + at[k], parts[k].first, parts[k].second);
+      std::vector<char> host;
+      auto put = [&](const void* p, size_t bytes) {
+        const size_t at = host.size();
+        host.resize(at + (bytes + 255) / 256 * 256, 0);
+        if (bytes) std::memcpy(host.data() + at, p, bytes);
+        return at;
+      };
+      auto putSegs = [&](const std::vector<int4>& v) { return put(v.data(), v.size() * sizeof(int4)); };
+      const size_t atRve = put(&rd, sizeof(rd)), atSegs = putSegs(segs);
+      size_t at[kLoads][3];
+      for (int q = 0; q < kLoads; q++) {
+        at[q][0] = putSegs(s2[q]);
+        at[q][1] = putSegs(c3[q]);
+        at[q][2] = putSegs(c2[q]);
+      }
+      const size_t atTiles = put(tiles.data(), tiles.size() * sizeof(ResTile));
       // (after the tables: the record and exchange buffer of resident runs)
       const size_t resBytes = resTiles_ ? 256 + 2 * (size_t)resXpar_ : 0;
-      char* blk = (char*)alloc(at[6] + resBytes);
-      dRve_ = (RveDev*)blk;
-      dSegs_ = (int4*)(blk + at[1]);
-      dSegs2_ = (int4*)(blk + at[2]);
-      dSegsC3_ = (int4*)(blk + at[3]);
-      dSegsC2_ = (int4*)(blk + at[4]);
-      dResTiles_ = (ResTile*)(blk + at[5]);
+      char* blk = (char*)alloc(host.size() + resBytes);
+      dRve_ = (RveDev*)(blk + atRve);
+      dSegs_ = (int4*)(blk + atSegs);
+      for (int q = 0; q < kLoads; q++) {
+        Segments& g = segsFor_[q];
+        g.n = (int)s2[q].size();
+        g.n3 = (int)c3[q].size();
+        g.n2 = (int)c2[q].size();
+        g.d = (int4*)(blk + at[q][0]);
+        g.d3 = (int4*)(blk + at[q][1]);
+        g.d2 = (int4*)(blk + at[q][2]);
+      }
+      dResTiles_ = (ResTile*)(blk + atTiles);
       if (resTiles_) {
-        dResCtl_ = (ResCtl*)(blk + at[6]);
-        dXch_ = blk + at[6] + 256;
-        launch_fill((double*)(blk + at[6]), resBytes / 8, 0.0, stream_);
+        dResCtl_ = (ResCtl*)(blk + host.size());
+        dXch_ = blk + host.size() + 256;
+        launch_fill((double*)(blk + host.size()), resBytes / 8, 0.0, stream_);
       }
       h2d(blk, host.data(), host.size());
     }
@@ -454,12 +473,17 @@ bool Solver::residentFits(long n) {
     return false;
   }
   if (++resRun_ == 0) resRun_ = 1;
-  return inRoom_->enter(&room_, resRun_, cus_);
+  return enterRoom(resRun_, n) == 0;
 }
 
-// Before launches of the other kernels: the handle is at work.
-void Solver::enterRoom() {
-  if (inRoom_) inRoom_->enter(&room_, 0, cus_);
+// Before launches of n iterations: the handle is at work, with a resident run or
+// (0) on the other kernels, whose segments are those for the handles at work.
+int Solver::enterRoom(unsigned run, long n) {
+  int at = 1;
+  if (inRoom_ && run == 0 && (n <= 1 || !tileSingles_)) inRoom_->work(&room_);
+  else if (inRoom_) at = inRoom_->enter(&room_, run, cus_);
+  load_ = tileSingles_ ? std::clamp(at, 1, kLoads) - 1 : 0;
+  return at;
 }
 
 void Solver::launchResidentRun(long n) {
@@ -535,7 +559,7 @@ bool Solver::settled() {
     // U and V are torn: no call uses them until they are set again (the
     // stress fields are as in a new handle)
     lostFields_ = 15;
-    enterRoom();
+    enterRoom(0, 0);
     const size_t nC = (size_t)nX_ * nY_, nV = (size_t)(nX_ - 1) * (nY_ - 1);
     for (double* p : {f_.P, f_.tauXX, f_.tauYY, f_.tauXYav, f_.J2})
       launch_fill(p, nC, 0.0, stream_);
@@ -785,17 +809,18 @@ void Solver::noteTimed(const std::pair<hipEvent_t, hipEvent_t>& ev, TimedKind ki
 // and written to the other, so after an odd number of such launches the
 // other buffer is current (flipV).
 void Solver::launchMulti(int q) {
+  const Segments& g = segsFor_[load_];
   const bool timed = sampleEvery_ > 0 && (launchCount_ % sampleEvery_) == 0;
   std::pair<hipEvent_t, hipEvent_t> ev{};
   if (timed) ev = takeTimingEvents();
   if (ipl_ == 2)
-    launch_march2(dRve_, dSegs2_, nSegs2_, iterMode(), cur_, vIdx_ ^ (q & 1), stream_,
+    launch_march2(dRve_, g.d, g.n, iterMode(), cur_, vIdx_ ^ (q & 1), stream_,
                   timed ? ev.first : nullptr, timed ? ev.second : nullptr, true);
   else if (wide_)
-    launch_wide(ipl_, dRve_, dSegs2_, nSegs2_, cur_, vIdx_ ^ (q & 1), stream_,
+    launch_wide(ipl_, dRve_, g.d, g.n, cur_, vIdx_ ^ (q & 1), stream_,
                 timed ? ev.first : nullptr, timed ? ev.second : nullptr);
   else
-    launch_chain(ipl_, dRve_, dSegs2_, nSegs2_, iterMode(), cur_, vIdx_ ^ (q & 1), stream_,
+    launch_chain(ipl_, dRve_, g.d, g.n, iterMode(), cur_, vIdx_ ^ (q & 1), stream_,
                  timed ? ev.first : nullptr, timed ? ev.second : nullptr, stageWaves_);
   cur_ ^= 1;
   stressStale_ = true;
@@ -889,7 +914,7 @@ void Solver::dropPlainGraph() {
 void Solver::iterateLaunches(long n) {
   if (n > 0) {
     lastResident_ = false;
-    enterRoom();
+    enterRoom(0, n);
   }
   n -= replayPlain(n);
   if (!multiIter_ || (stress64_ && !multi64())) {
@@ -905,11 +930,11 @@ void Solver::iterateLaunches(long n) {
   for (long q = 0; q < d; q++) launchMulti((int)(q & 1));
   // four closing iterations run as a three-iteration launch and the single,
   // three as a two-iteration launch and the single (the same results)
-  if (singles == 4 && nSegsC3_ > 0) {
+  if (singles == 4 && segsFor_[load_].n3 > 0) {
     launchClose(3, (int)(d & 1));
     d++;
     singles = 1;
-  } else if (singles == 3 && nSegsC2_ > 0) {
+  } else if (singles == 3 && segsFor_[load_].n2 > 0) {
     launchClose(2, (int)(d & 1));
     d++;
     singles = 1;
@@ -922,11 +947,12 @@ void Solver::iterateLaunches(long n) {
 // closing a run of multi-iteration launches; V is read from buffer
 // vIdx_ ^ q and written to the other, as in launchMulti.
 void Solver::launchClose(int ns, int q) {
+  const Segments& g = segsFor_[load_];
   if (ns == 3)
-    launch_chain(3, dRve_, dSegsC3_, nSegsC3_, iterMode(), cur_, vIdx_ ^ q, stream_, nullptr,
+    launch_chain(3, dRve_, g.d3, g.n3, iterMode(), cur_, vIdx_ ^ q, stream_, nullptr,
                  nullptr, 1);
   else
-    launch_march2(dRve_, dSegsC2_, nSegsC2_, iterMode(), cur_, vIdx_ ^ q, stream_, nullptr,
+    launch_march2(dRve_, g.d2, g.n2, iterMode(), cur_, vIdx_ ^ q, stream_, nullptr,
                   nullptr, true);
   cur_ ^= 1;
   stressStale_ = true;
@@ -991,7 +1017,7 @@ std::string Solver::kernelName(TimedKind kind) const {
             : wide_ ? "k_wide<" + std::to_string(ipl_) + ">"
                     : std::string(f32 ? "k_chain<float, float, " : "k_chain<double, double, ") +
                           std::to_string(ipl_) + ", " + std::to_string(stageWaves_) + ">") +
-           " rows=" + std::to_string(marchRows_) + " segments=" + std::to_string(nSegs2_) +
+           " rows=" + std::to_string(marchRows_) + " segments=" + std::to_string(segsFor_[0].n) +
            " (per iteration)";
   if (marchRows_ > 0 && !tileSingles_)
     return std::string(f32 ? "k_march<float, float>" : "k_march<double, double>") +

@@ -178,14 +178,18 @@ class Solver {
   int ipl_ = 1;                     // iterations per launch: 1, 2 (pairs), 3 or 4 (chains)
   bool wide_ = false;               // chains on two columns per lane (split scheme)
   int stageWaves_ = 1;              // chains: waves side by side per stage
-  int nSegs2_ = 0;
-  int4* dSegs2_ = nullptr;
-  // segments of the three- and two-iteration launches that close a run of a
-  // four- or three-iteration shape (chains of three waves, 42 rows; wave
-  // pairs, 26 rows)
-  int nSegsC3_ = 0, nSegsC2_ = 0;
-  int4* dSegsC3_ = nullptr;
-  int4* dSegsC2_ = nullptr;
+  // Segments of the multi-iteration launches, and of the three- and
+  // two-iteration ones that close a run of a four- or three-iteration shape
+  // (chains of three waves, 42 rows; wave pairs, 26 rows).  Grids below 1024^2 on
+  // the automatic shape have them for one, two, and
+  // three handles and more at work.
+  struct Segments {
+    int rows = 0, n = 0, n3 = 0, n2 = 0;
+    int4 *d = nullptr, *d3 = nullptr, *d2 = nullptr;
+  };
+  static constexpr int kLoads = 3;
+  Segments segsFor_[kLoads];
+  int load_ = 0;                    // the ones in use
   bool tileSingles_ = false;        // single iterations on the tile kernel
   int vIdx_ = 0;                    // velocity buffer holding the current V
   void flipV();                     // the other velocity buffer becomes current
@@ -211,7 +215,7 @@ class Solver {
   int resSkip_ = 0;                 // runs to take the other kernels after a late start
   void planResident(std::vector<ResTile>& tiles);
   bool residentFits(long n);
-  void enterRoom();
+  int enterRoom(unsigned run, long n);
   void launchResidentRun(long n);
   void noteRuns();                  // drop the runs known to have completed
   bool settled();                   // after the stream is synchronised

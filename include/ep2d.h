@@ -236,8 +236,9 @@ int ep2d_get_mask(ep2d_handle* h, unsigned char* host, size_t count);
 
 /* ---- step-level entry points (the pieces ComputeEffParams is made of) ----*/
 /* n iterations of the handle's scheme, no residual checks (:389-399).  The work
- * is queued; on a handle with its own stream, a call of fewer than 16
- * iterations (and ep2d_apply_affine) behind a resident run waits for it
+ * is queued.  On a handle with its own stream, what cannot run resident (a call
+ * of fewer than 16 iterations, one beside other handles that leave no room,
+ * ep2d_apply_affine) waits for a resident run of the handle before it
  * (ep2d_diag_resident). */
 int ep2d_iterate(ep2d_handle* h, long n);
 /* U += affine field of the macro strain increment (:370-381), on device. */
