@@ -209,12 +209,19 @@ struct ResCtl {
 struct ResLimits {
   unsigned arriveTicks = 25000000u, polls = 1u << 20;
 };
-// how a launch went: run, or ended with the fields untouched because its tiles
-// did not all start in time; lost: a wait inside the run ended at its bound
+// how a launch went: run, or ended with the fields untouched because launches
+// that were running left it no room or its tiles did not all start in time; lost: a wait inside the run ended at its bound
 // (the fields are not valid); after: an earlier launch did not run
-constexpr unsigned kResGo = 1, kResLate = 2, kResLost = 3, kResAfter = 4;
+constexpr unsigned kResGo = 1, kResLate = 2, kResLost = 3, kResAfter = 4, kResNoRoom = 5;
 constexpr long kResMinIters = 16;  // shorter runs take the other kernels
 constexpr int kResMinSide = 16;
+// Room of resident tiles: `whole` tiles take a CU each, two `half` ones share
+// one.  Half tiles spread one to a CU while CUs are free, so beside whole tiles
+// each counts as a CU: then every tile of the launches let in finds its place,
+// in whatever order they start and end.
+__host__ __device__ inline bool resident_fits(unsigned cus, unsigned half, unsigned whole) {
+  return whole == 0 ? half <= 2 * cus : half + whole <= cus;
+}
 struct ResLaunch {
   int mode;                 // scheme (1 or 2)
   ResShape shape;
@@ -228,6 +235,8 @@ struct ResLaunch {
   unsigned tag0;            // tags tag0 + 1 .. tag0 + iters, none used before
   ResCtl* ctl;
   ResLimits limits;
+  unsigned half, whole;     // the launch's tiles by what they take of a CU
+  unsigned cus;
   unsigned run;             // the number the launch is known by (not 0)
   unsigned* told;           // two pinned host words: receive `run` if it ran, else how it failed
 };

@@ -33,16 +33,18 @@
 // hence read k-1's (all its waves: a barrier stands between).
 //
 // Every wait ends.  A tile waits for its neighbours, so all tiles of a launch
-// must run at once, and no tile starts before all have arrived.  The host lets
-// only so many launches of this process in as find their places together
-// (DeviceRoom): tiles of the split two-row shape take half a CU's registers (118
-// a lane at eight waves), the others (146 to 204) a CU each.  Other work on the
-// device gives its places up as it ends.  If the tiles have not all arrived
-// within a quarter second (another process holds the GPU, or work this library
-// does not know of), the launch ends without having changed anything and says
-// so, those queued behind it do the same, and the caller takes the other kernels;
-// until then the tiles that have arrived hold their places.  Waits inside the
-// run are bounded too.
+// must run at once, and no tile starts before all have arrived.  The first
+// workgroup of a launch to run counts its tiles among those in flight on the
+// device and goes on only if all of them find their places together
+// (resident_fits): tiles of the split two-row shape take half a CU's registers
+// (118 a lane at eight waves), the others (146 to 204) a CU each.  The host does
+// not launch what it knows to find no room (DeviceRoom).  Other work on the
+// device gives its places up as it ends.  If there is no room, or the tiles have
+// not all arrived within a quarter second (another process holds the GPU, or
+// work this library does not know of), the launch ends without having changed
+// anything and says so, those queued behind it do the same, and the caller takes
+// the other kernels; until then the tiles that have arrived hold their places.
+// Waits inside the run are bounded too.
 #include "ep2d_internal.h"
 #include "ep2d_march.h"
 
@@ -51,6 +53,10 @@
 namespace ep2d {
 
 namespace {
+
+// resident tiles in flight on this device: half-CU ones in the low 16 bits,
+// whole ones above
+__device__ unsigned g_resInUse;
 
 __device__ __forceinline__ unsigned ald(unsigned* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -65,13 +71,17 @@ __device__ __forceinline__ unsigned acas(unsigned* p, unsigned from, unsigned to
 }
 
 // Arrival of one workgroup (its first thread): the state all of them see.  The
-// first to arrive decides: it waits for the others and lets the run go, or
-// ends it.  (The others' bound is longer: it only serves
+// first to arrive decides: it counts the tiles in, waits for the others and
+// lets the run go, or ends it.  (The others' bound is longer: it only serves
 // if the first never decides.)
-__device__ unsigned res_arrive(ResCtl* c, unsigned tiles, unsigned ticks) {
+__device__ unsigned res_arrive(ResCtl* c, unsigned tiles, unsigned ticks, unsigned need,
+                               unsigned cus) {
   const unsigned long long t0 = wall_clock64();
   if (aadd(&c->arrive, 1u) == 0) {
-    unsigned how = ald(&c->failed) != 0u ? kResAfter : ticks ? kResGo : kResLate;
+    const unsigned use = aadd(&g_resInUse, need) + need;
+    unsigned how = ald(&c->failed) != 0u ? kResAfter
+                   : !resident_fits(cus, use & 0xffffu, use >> 16) ? kResNoRoom
+                   : ticks ? kResGo : kResLate;
     while (how == kResGo && ald(&c->arrive) < tiles) {
       if (wall_clock64() - t0 > ticks) how = kResLate;
       __builtin_amdgcn_s_sleep(1);
@@ -90,12 +100,15 @@ __device__ unsigned res_arrive(ResCtl* c, unsigned tiles, unsigned ticks) {
   }
 }
 
-// Departure: the last workgroup clears the record for the next launch and tells
-// the host how this one went.
-__device__ void res_depart(ResCtl* c, unsigned tiles, unsigned run, unsigned* told) {
+// Departure: the last workgroup counts the tiles out (also those of a launch that
+// did not run), clears the record for the next launch and tells the host how
+// this one went.
+__device__ void res_depart(ResCtl* c, unsigned tiles, unsigned need, unsigned run,
+                           unsigned* told) {
   __builtin_amdgcn_s_waitcnt(0);
   if (aadd(&c->depart, 1u) + 1 != tiles) return;
   const unsigned s = ald(&c->state);
+  aadd(&g_resInUse, 0u - need);
   __hip_atomic_store(&c->arrive, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __hip_atomic_store(&c->depart, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __hip_atomic_store(&c->state, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -808,8 +821,8 @@ constexpr int res_waves() {
 template <typename CT, typename VT, int R, int T, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(res_waves<CT, R>()))) void k_resident(
     const RveDev* __restrict__ rves, const ResTile* __restrict__ tiles, int parity, int vpar,
-    int n, const char* xch, unsigned xpar, unsigned tag0, ResCtl* ctl, ResLimits lim, unsigned run,
-    unsigned* told) {
+    int n, const char* xch, unsigned xpar, unsigned tag0, ResCtl* ctl, ResLimits lim, unsigned need,
+    unsigned cus, unsigned run, unsigned* told) {
   using Lds = ResLds<CT, VT, R, T, NW>;
   __shared__ Lds lds;
   const int v = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -823,7 +836,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(res_wav
       (&lds.zeroV[0][0][0])[2 * threadIdx.x + 1] = (VT)0;
     }
   }
-  if (threadIdx.x == 0) lds.state = res_arrive(ctl, gridDim.x, lim.arriveTicks);
+  if (threadIdx.x == 0) lds.state = res_arrive(ctl, gridDim.x, lim.arriveTicks, need, cus);
   __syncthreads();
   if (lds.state == kResGo) {
     bool lost = false;
@@ -863,7 +876,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(res_wav
     if (__any(lost) && (threadIdx.x & 63) == 0) acas(&ctl->state, kResGo, kResLost);
   }
   __syncthreads();
-  if (threadIdx.x == 0) res_depart(ctl, gridDim.x, run, told);
+  if (threadIdx.x == 0) res_depart(ctl, gridDim.x, need, run, told);
 }
 
 // the kernel of a scheme and a tile shape
@@ -964,12 +977,14 @@ void launch_resident(const ResLaunch& a, hipStream_t s, hipEvent_t e0, hipEvent_
   const dim3 grid((unsigned)a.tiles), block(64 * a.shape.waves);
   res_dispatch(a.mode, a.shape, [&](auto kern) {
     const char* xch = a.xch;
+    const unsigned need = a.half | a.whole << 16;
     if (e0)
       hipExtLaunchKernelGGL(kern, grid, block, 0, s, e0, e1, 0, a.rves, a.list, a.parity, a.vpar,
-                            a.iters, xch, a.xpar, a.tag0, a.ctl, a.limits, a.run, a.told);
+                            a.iters, xch, a.xpar, a.tag0, a.ctl, a.limits, need, a.cus, a.run,
+                            a.told);
     else
       hipLaunchKernelGGL(kern, grid, block, 0, s, a.rves, a.list, a.parity, a.vpar, a.iters, xch,
-                         a.xpar, a.tag0, a.ctl, a.limits, a.run, a.told);
+                         a.xpar, a.tag0, a.ctl, a.limits, need, a.cus, a.run, a.told);
     return 0;
   });
   EP2D_HIP(hipGetLastError());

@@ -11,14 +11,6 @@
 
 namespace ep2d {
 
-// Room of resident tiles: `whole` tiles take a CU each, two `half` ones share
-// one.  Half tiles spread one to a CU while CUs are free, so beside whole tiles
-// each counts as a CU: then every tile of the launches let in finds its place,
-// in whatever order they start and end.
-inline bool resident_fits(unsigned cus, unsigned half, unsigned whole) {
-  return whole == 0 ? half <= 2 * cus : half + whole <= cus;
-}
-
 // What one handle has on a device.  Its fields are the room's while the handle
 // is in it.
 struct RoomUser {
@@ -39,6 +31,7 @@ inline bool run_ended(const unsigned* told, unsigned run) {
 // The handles of this process on one device.
 class DeviceRoom {
  public:
+  static constexpr size_t kQueues = 4;  // HIP's default (GPU_MAX_HW_QUEUES)
   static DeviceRoom& of(int device) {
     // never destroyed: handles may outlive static objects
     static std::mutex* m = new std::mutex;
@@ -57,20 +50,30 @@ class DeviceRoom {
   }
   // Before work of `me` is enqueued: 0 if the resident run `run` (0: none) may be
   // launched, else the handles at work, `me` among them (counted to 3).  It may
-  // be if all handles at work fit the device with their resident tiles (one
-  // that has no such shape leaves no room).
+  // be if it fits the device beside the resident tiles of the others that can
+  // run at once with it, the largest (a handle that has no such shape leaves no
+  // room): the process has kQueues hardware queues, and launches of streams
+  // that share one run one after another.  The launch itself counts exactly.
   int enter(RoomUser* me, unsigned run, unsigned cus) {
     const std::lock_guard<std::mutex> lock(m_);
-    unsigned half = me->half, whole = me->whole;
     int n = 1;
     bool all = run != 0;
+    std::vector<const RoomUser*> at;
     for (RoomUser* u : users_) {
       if (!all && n >= 3) break;
       if (u == me || !busy(*u)) continue;
       n++;
-      half += u->half;
-      whole += u->whole;
+      at.push_back(u);
       all = all && u->half + u->whole > 0;
+    }
+    if (at.size() >= kQueues)
+      std::sort(at.begin(), at.end(), [](const RoomUser* a, const RoomUser* b) {
+        return a->half + 2 * a->whole > b->half + 2 * b->whole;
+      });
+    unsigned half = me->half, whole = me->whole;
+    for (size_t k = 0; k < std::min(at.size(), kQueues - 1); k++) {
+      half += at[k]->half;
+      whole += at[k]->whole;
     }
     all = all && resident_fits(cus, half, whole);
     // (a run that is turned down leaves those before it in the entry; the other

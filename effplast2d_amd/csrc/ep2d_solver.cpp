@@ -194,7 +194,7 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
   EP2D_HIP(hipGetDeviceCount(&ndev));
   if (device_ < 0 || device_ >= ndev) throw ArgError("device index out of range");
   EP2D_HIP(hipSetDevice(device_));
-  cus_ = (unsigned)device_cus(device_);
+  cus_ = resCus_ = (unsigned)device_cus(device_);
   if (stream) {
     stream_ = stream;
     ownStream_ = false;
@@ -508,6 +508,9 @@ void Solver::launchResidentRun(long n) {
   a.tag0 = resTag_;
   a.ctl = dResCtl_;
   a.limits = resLimits_;
+  a.half = room_.half;
+  a.whole = room_.whole;
+  a.cus = resCus_;
   a.run = resRun_;
   a.told = hResTold_;
   launch_resident(a, stream_, timed ? ev.first : nullptr, timed ? ev.second : nullptr);
@@ -552,9 +555,9 @@ bool Solver::settled() {
       k++;
     }
   }
-  const bool lost = how != kResLate;
+  const bool lost = how != kResLate && how != kResNoRoom;
   resCounts_[lost ? 2 : 1]++;
-  resSkip_ = 256;
+  if (how != kResNoRoom) resSkip_ = 256;
   if (lost) {
     // U and V are torn: no call uses them until they are set again (the
     // stress fields are as in a new handle)
@@ -593,15 +596,16 @@ void Solver::settle() {
 }
 
 // Counts of the handle's resident runs (completed, turned away or late, lost),
-// and the bounds and exchange tag of its later ones (negative: unchanged).
+// and the bounds, exchange tag and room of its later ones (negative: unchanged).
 void Solver::diagResident(const long long* limits, long long* counts) {
   settleRun();
   for (int k = 0; counts && k < 3; k++) counts[k] = resCounts_[k];
   if (!limits || resTiles_ == 0) return;
-  for (int k = 0; k < 3; k++)
+  for (int k = 0; k < 4; k++)
     if (limits[k] > 0xffffffffLL) throw ArgError("ep2d_diag_resident: limit out of range");
   if (limits[0] >= 0) resLimits_.arriveTicks = (unsigned)limits[0];
   if (limits[1] >= 0) resLimits_.polls = (unsigned)limits[1];
+  if (limits[3] >= 0) resCus_ = (unsigned)limits[3];
   if (limits[2] >= 0) {
     // (no word of the buffer carries a later tag)
     EP2D_HIP(hipSetDevice(device_));

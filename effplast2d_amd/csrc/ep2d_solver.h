@@ -211,6 +211,7 @@ class Solver {
   };
   std::deque<ResRun> resRuns_;
   ResLimits resLimits_;
+  unsigned resCus_ = 0;             // CUs the launches count on
   long long resCounts_[3] = {0, 0, 0};  // completed, turned away or late, lost
   int resSkip_ = 0;                 // runs to take the other kernels after a late start
   void planResident(std::vector<ResTile>& tiles);

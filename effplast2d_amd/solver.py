@@ -226,10 +226,10 @@ class EffPlast2D:
     def sync(self):
         check(lib().ep2d_sync(self._h))
 
-    def diag_resident(self, arrive_ticks=-1, polls=-1, tag=-1):
+    def diag_resident(self, arrive_ticks=-1, polls=-1, tag=-1, cus=-1):
         """Resident runs of the handle so far: completed, not started, lost; the
         arguments set limits of its later runs (ep2d_diag_resident)."""
-        lim = (C.c_longlong * 3)(arrive_ticks, polls, tag)
+        lim = (C.c_longlong * 4)(arrive_ticks, polls, tag, cus)
         cnt = (C.c_longlong * 3)()
         check(lib().ep2d_diag_resident(self._h, lim, cnt))
         return tuple(cnt)

@@ -297,14 +297,15 @@ int ep2d_diag_chain_order(const int* segs, int n, int stageWaves, const int* dim
 /* Diagnostic, no counterpart in the reference: the resident runs of a handle
  * (runs of 16 iterations and more of a grid that fits on the chip, in one
  * launch).  counts (3 words, may be NULL) receives the runs completed, those
- * whose workgroups did not all start in time (their iterations took the other
+ * that found no room or whose workgroups did not all start in time (their iterations took the other
  * kernels: the same results) and those that lost a wait inside the run.
  * After a lost one (reported once as EP2D_ERR_HIP) the calls that use the state
  * return EP2D_ERR_STATE until Ux, Uy, Vx and Vy have been set.
- * limits (3 words, may be NULL) sets, for the handle's later runs, [0] the
+ * limits (4 words, may be NULL) sets, for the handle's later runs, [0] the
  * ticks of 10 ns a launch waits for its workgroups (0: it never starts), [1]
  * the polls of about a microsecond a wait inside the run takes, [2] the number
- * its exchanges are counted on from (32 bits); negative: unchanged.  For tests
+ * its exchanges are counted on from (32 bits), [3] the CUs a launch finds room
+ * on; negative: unchanged.  For tests
  * of the paths a busy device takes. */
 int ep2d_diag_resident(ep2d_handle* h, const long long* limits, long long* counts);
 /* Analytic static solution of the single-pore problem beside the numerical

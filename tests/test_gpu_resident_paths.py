@@ -365,3 +365,45 @@ def test_many_handles_are_no_slower_than_tiles():
     mine, tiles = run(), run(tileRows=8)
     print(f"{mine * 1e3:.1f} ms, tiles {tiles * 1e3:.1f} ms", flush=True)
     assert mine < 1.1 * tiles
+
+
+@pytest.mark.parametrize("mode,nX", [("fp64", 125), ("split", 200)])
+def test_runs_that_find_no_room(mode, nX):
+    """A launch that finds other tiles in its room ends at once; the next run is
+    tried again."""
+    print(f"no room {mode} nX={nX}", flush=True)
+    pa, init = _case(nX, mode, 17 + nX)
+    steps = (33, 16, 18)
+    with EffPlast2D(pa, nX, nTasks=3, mode=mode) as g:
+        _start(g, init)
+        g.diag_resident(cus=1)
+        for n in steps:
+            g.iterate(n)
+            g.sync()
+        assert g.diag_resident(cus=256) == (0, 3, 0)
+        g.iterate(20)
+        a = {k: g.get(k) for k in FIELDS}
+        assert g.diag_resident() == (1, 3, 0)
+    _same(a, _tiles(nX, mode, pa, init, sum(steps) + 20))
+
+
+@pytest.mark.parametrize("mode,nX,k", [("fp64", 128, 8), ("split", 128, 16)])
+def test_small_handles_share_the_device(mode, nX, k):
+    """Handles whose tiles fit the device as far as they can run at once stay
+    resident side by side, however many are queued."""
+    print(f"{k} handles {mode} nX={nX}", flush=True)
+    cases = [_case(nX, mode, 80 + q) for q in range(k)]
+    hs = [EffPlast2D(pa, nX, nTasks=3, mode=mode) for pa, _ in cases]
+    try:
+        for h, (_, init) in zip(hs, cases):
+            _start(h, init)
+        for n in (700, 33):
+            for h in hs:
+                h.iterate(n)
+        for h in hs:
+            assert h.diag_resident() == (2, 0, 0)
+        for h, (pa, init) in list(zip(hs, cases))[::5]:
+            _same({f: h.get(f) for f in FIELDS}, _tiles(nX, mode, pa, init, 733))
+    finally:
+        for h in hs:
+            h.close()
