@@ -88,11 +88,13 @@ Batch::Batch(const ep2d_batch_options& opt) : opt_(opt) {
   EP2D_HIP(hipMemGetInfo(&freeB, &totalB));
   budget_ = opt_.memoryBudget ? opt_.memoryBudget : (size_t)(0.9 * (double)freeB);
   t0_ = std::chrono::steady_clock::now();
+  DeviceRoom::of(device_).join(&room_);
 }
 
 Batch::~Batch() {
   (void)hipSetDevice(device_);
   if (stream_) (void)hipStreamSynchronize(stream_);
+  DeviceRoom::of(device_).leave(&room_);
   active_.clear();
   dropGraphs();
   for (auto& e : evPending_) {
@@ -820,7 +822,21 @@ void Batch::resolveEvents() {
   }
 }
 
+namespace {
+struct AtWork {
+  DeviceRoom& room;
+  RoomUser* me;
+  AtWork(DeviceRoom& r, RoomUser* u) : room(r), me(u) { room.work(me, true); }
+  ~AtWork() { room.work(me, false); }
+};
+}  // namespace
+
 void Batch::step(int* nActive, int* nQueued) {
+  const AtWork at(DeviceRoom::of(device_), &room_);
+  advance(nActive, nQueued);
+}
+
+void Batch::advance(int* nActive, int* nQueued) {
   EP2D_HIP(hipSetDevice(device_));
   admit();
   if (!active_.empty()) {
@@ -908,9 +924,10 @@ void Batch::step(int* nActive, int* nQueued) {
 }
 
 void Batch::run() {
+  const AtWork at(DeviceRoom::of(device_), &room_);
   int a = 0, q = 0;
   do {
-    step(&a, &q);
+    advance(&a, &q);
   } while (a > 0 || q > 0);
 }
 

@@ -91,6 +91,7 @@ class Batch {
   static constexpr int kMaxGraphs = 6;
   static constexpr long kMinGraphLaunches = 16;  // shorter runs launch directly
 
+  void advance(int* nActive, int* nQueued);
   size_t estimateBytes(const ep2d_request& rq) const;
   void admit();
   void fail(Slot& sl, int status, const char* what);
@@ -120,6 +121,7 @@ class Batch {
   int device_ = 0;
   MemPool pool_;   // buffers of retired RVEs, reused by the next admissions
   hipStream_t stream_ = nullptr;
+  RoomUser room_;  // at work during a step: resident tiles leave it its share
   std::chrono::steady_clock::time_point t0_;
   std::deque<Job> queue_;
   std::vector<Slot> active_;

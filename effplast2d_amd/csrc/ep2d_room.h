@@ -1,5 +1,5 @@
-// ep2d_room.h -- which handles of this process are at work on a device, and
-// which of them may run resident (ep2d_resident.hip) side by side.
+// ep2d_room.h -- which handles and batches of this process are at work on a
+// device, and which handles may run resident (ep2d_resident.hip) side by side.
 #pragma once
 
 #include <algorithm>
@@ -11,15 +11,16 @@
 
 namespace ep2d {
 
-// What one handle has on a device.  Its fields are the room's while the handle
-// is in it.
+// What one handle, or batch, has on a device.  Its fields are the room's while the
+// handle is in it.
 struct RoomUser {
   hipStream_t stream = nullptr;      // its work
   unsigned half = 0, whole = 0;      // its resident tiles (0, 0: it has no such shape)
   const unsigned* told = nullptr;    // pinned words a resident run writes when it ends
   unsigned run = 0;                  // the resident run it has in flight (0: none)
   bool atWork = false;               // other work may be in flight
-  bool held = false;                 // its stream must not be asked (a capture is on)
+  bool held = false;                 // its stream must not be asked (a capture is on),
+                                     // or need not be (a batch in a step)
 };
 
 // The words: the last run that has completed, and how a run failed (0: none did).
@@ -28,7 +29,7 @@ inline bool run_ended(const unsigned* told, unsigned run) {
          __atomic_load_n(told + 1, __ATOMIC_ACQUIRE) != 0;
 }
 
-// The handles of this process on one device.
+// The handles and batches of this process on one device.
 class DeviceRoom {
  public:
   static constexpr size_t kQueues = 4;  // HIP's default (GPU_MAX_HW_QUEUES)
@@ -51,20 +52,27 @@ class DeviceRoom {
   // Before work of `me` is enqueued: 0 if the resident run `run` (0: none) may be
   // launched, else the handles at work, `me` among them (counted to 3).  It may
   // be if it fits the device beside the resident tiles of the others that can
-  // run at once with it, the largest (a handle that has no such shape leaves no
-  // room): the process has kQueues hardware queues, and launches of streams
-  // that share one run one after another.  The launch itself counts exactly.
+  // run at once with it, the largest: the process has kQueues hardware queues,
+  // and launches of streams that share one run one after another.  The launch
+  // itself counts exactly.
+  // Resident tiles keep their CUs for the whole run, so beside work that is not
+  // resident (a batch, a larger grid) they take a quarter of the device at most.
+  // A batch of 20 split 1024^2 (124 ms a pass alone) beside a handle that runs
+  // intervals of 500 iterations: FP64 128^2 (48 CUs) resident 142 ms a pass and
+  // 2.7 ms an interval, on the chains 134 and 11; FP64 512^2 (240 CUs) resident
+  // 612 and 3.2, on the chains 139 and 16 (on tiles, each iteration a launch,
+  // 151 and 15).
   int enter(RoomUser* me, unsigned run, unsigned cus) {
     const std::lock_guard<std::mutex> lock(m_);
     int n = 1;
-    bool all = run != 0;
+    bool all = run != 0, shared = false;
     std::vector<const RoomUser*> at;
     for (RoomUser* u : users_) {
-      if (!all && n >= 3) break;
+      if (run == 0 && n >= 3) break;
       if (u == me || !busy(*u)) continue;
       n++;
       at.push_back(u);
-      all = all && u->half + u->whole > 0;
+      shared = shared || u->half + u->whole == 0;
     }
     if (at.size() >= kQueues)
       std::sort(at.begin(), at.end(), [](const RoomUser* a, const RoomUser* b) {
@@ -75,7 +83,7 @@ class DeviceRoom {
       half += at[k]->half;
       whole += at[k]->whole;
     }
-    all = all && resident_fits(cus, half, whole);
+    all = all && (shared ? half + whole <= cus / 4 : resident_fits(cus, half, whole));
     // (a run that is turned down leaves those before it in the entry; the other
     // kernels' launches, run 0, come when the handle has none in flight)
     if (all || run == 0) me->run = run;
@@ -87,6 +95,11 @@ class DeviceRoom {
     const std::lock_guard<std::mutex> lock(m_);
     me->run = 0;
     me->atWork = true;
+  }
+  // A batch's step.
+  void work(RoomUser* me, bool on) {
+    const std::lock_guard<std::mutex> lock(m_);
+    me->atWork = me->held = on;
   }
   void hold(RoomUser* me, bool on) {
     const std::lock_guard<std::mutex> lock(m_);

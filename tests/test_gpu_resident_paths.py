@@ -11,7 +11,7 @@ import pytest
 # torch before the library: one HIP runtime in the process
 import torch  # noqa: F401
 
-from effplast2d_amd import EffPlast2D, Ep2dError
+from effplast2d_amd import Batch, EffPlast2D, Ep2dError
 from tests.pairs import PLASTIC_FIELDS, STATE_FIELDS, STRESS_FIELDS, make_pa, random_state
 
 pytestmark = pytest.mark.gpu
@@ -407,3 +407,41 @@ def test_small_handles_share_the_device(mode, nX, k):
     finally:
         for h in hs:
             h.close()
+
+
+@pytest.mark.parametrize("nX,resident", [(512, 0), (128, 4)])
+def test_a_batch_keeps_its_share(nX, resident):
+    """Beside a batch in a step a handle runs resident if its tiles take a quarter
+    of the device at most (240 and 48 CUs here), else its iterations take the
+    chains; both end with their results."""
+    print(f"batch beside a handle {nX}", flush=True)
+    pa, init = _case(nX, "fp64", 6)
+    bpa = make_pa(1024, nPores=1, porosity=0.02)
+    state = {}
+
+    def batch():
+        with Batch(mode="split", checkInterval=500) as eng:
+            for tag in range(8):
+                eng.submit(bpa, nX=1024, nTasks=1, nIter=6000, eIter=1e-30, initLoad=-1e-3,
+                           loadType=[1.0, 1.0, 0.0], tag=tag)
+            state["started"] = True
+            eng.run()
+            state["out"] = eng.poll()
+
+    th = threading.Thread(target=batch)
+    with EffPlast2D(pa, nX, nTasks=3, mode="fp64") as g:
+        _start(g, init)
+        th.start()
+        while "started" not in state:
+            time.sleep(0.001)
+        time.sleep(0.05)
+        for _ in range(4):
+            g.iterate(25)
+            g.sync()
+        busy = th.is_alive()
+        a = {k: g.get(k) for k in FIELDS}
+        runs = g.diag_resident()
+        th.join()
+    assert busy and runs == (resident, 0, 0)
+    assert [r["status"] for r in state["out"]] == [0] * 8
+    _same(a, _tiles(nX, "fp64", pa, init, 100))
