@@ -96,6 +96,12 @@ class DeviceRoom {
     me->run = 0;
     me->atWork = true;
   }
+  // The stream of `me` has been waited for.
+  void idle(RoomUser* me) {
+    const std::lock_guard<std::mutex> lock(m_);
+    me->run = 0;
+    me->atWork = false;
+  }
   // A batch's step.
   void work(RoomUser* me, bool on) {
     const std::lock_guard<std::mutex> lock(m_);

@@ -121,13 +121,20 @@ void* Solver::hostAlloc(size_t bytes) {
 template <typename T>
 void Solver::h2d(T* dst, const T* src, size_t n) {
   EP2D_HIP(hipMemcpyAsync(dst, src, n * sizeof(T), hipMemcpyHostToDevice, stream_));
-  EP2D_HIP(hipStreamSynchronize(stream_));
+  waitStream();
 }
 
 template <typename T>
 void Solver::d2h(T* dst, const T* src, size_t n) {
   EP2D_HIP(hipMemcpyAsync(dst, src, n * sizeof(T), hipMemcpyDeviceToHost, stream_));
+  waitStream();
+}
+
+// The handle's work is done (and seen to be by the other handles, which would
+// have to ask the stream).
+void Solver::waitStream() {
   EP2D_HIP(hipStreamSynchronize(stream_));
+  if (inRoom_) inRoom_->idle(&room_);
 }
 
 // EffPlast2D::EffPlast2D, EffPlast2D.cu:1541-1612.
@@ -290,6 +297,7 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
   const bool autoShape = fused && ownStream_ && opt_.tileRows == 0 && opt_.marchRows == 0 &&
                          opt_.itersPerLaunch == 0 && opt_.laneColumns == 0 &&
                          opt_.stageWaves == 0;
+  int places = 0;  // workgroups of the automatic chains the device holds at once
   if (fused && opt_.tileRows == 0 && opt_.marchRows == 0 && opt_.itersPerLaunch == 0) {
     // automatic shape for one RVE, from one-RVE measurements: four-stage
     // chains with two waves per stage (four iterations per launch, in the
@@ -310,7 +318,10 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
                         !(mode_ == EP2D_MODE_FP64 && opt_.laneColumns == 2);
     if (chains) {
       int rows = n <= 2048 ? 48 : 96;
-      if (n <= 1024) rows = chain_rows(nX, nY, chain_resident(4, 2, mode_ == EP2D_MODE_SPLIT));
+      if (n <= 1024) {
+        places = chain_resident(4, 2, mode_ == EP2D_MODE_SPLIT);
+        rows = chain_rows(nX, nY, places);
+      }
       opt_.marchRows = rows;
       opt_.itersPerLaunch = 4;
       if (opt_.laneColumns != 2 && opt_.stageWaves == 0) opt_.stageWaves = 2;
@@ -348,7 +359,8 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
       const int2 dims = make_int2(nX, nY);
       const bool f32 = mode_ == EP2D_MODE_SPLIT;
       const bool ordered = multiIter_ && ipl_ >= 3 && !wide_;
-      const int res = ordered ? chain_resident(ipl_, stageWaves_, f32) : 0;
+      const int res = !ordered ? 0 : tileSingles_ ? places : chain_resident(ipl_, stageWaves_, f32);
+      const int res3 = ipl_ == 4 ? chain_resident(3, 1, f32) : 0;
       const int loads = tileSingles_ ? kLoads : 1;
       for (int q = 0; q < loads && multiIter_; q++) {
         // the heights for one, two, and three handles and more at work: segments
@@ -377,7 +389,6 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
         march2_segments(nX, nY, r2, 0, c2[q].data());
         if (ipl_ == 4) {
           const int raw3 = chain_segments(3, nX, nY, r3, 0, nullptr, 1);
-          const int res3 = chain_resident(3, 1, f32);
           c3[q].resize((size_t)chain_work_order(nullptr, raw3, 1, &dims, res3, nullptr));
           chain_segments(3, nX, nY, r3, 0, c3[q].data(), 1);
           chain_work_order(c3[q].data(), raw3, 1, &dims, res3, c3[q].data());
@@ -579,7 +590,7 @@ void Solver::settleRun() {
   if (!resRuns_.empty()) noteRuns();
   if (resRuns_.empty()) return;
   EP2D_HIP(hipSetDevice(device_));
-  EP2D_HIP(hipStreamSynchronize(stream_));
+  waitStream();
   settled();
 }
 
@@ -1036,7 +1047,7 @@ std::string Solver::kernelName(TimedKind kind) const {
 
 void Solver::sync() {
   settleRun();
-  EP2D_HIP(hipStreamSynchronize(stream_));
+  waitStream();
 }
 
 // Stress fields as the reference holds them after the loop: the trial stress
@@ -1553,7 +1564,7 @@ void Solver::runJob(ep2d_result* out) {
       if (tsAtCheck()) {
         do {
           tsCheckLaunch();
-          EP2D_HIP(hipStreamSynchronize(stream_));
+          waitStream();
         } while (!settled());
         tsCheckFinish();
       }
@@ -1757,7 +1768,7 @@ const void* Solver::fieldDevice(int field) {
     case EP2D_FIELD_VY: p = r_.Vy; break;
     default: throw ArgError("K and G are not stored on the device (the mask selects them)");
   }
-  EP2D_HIP(hipStreamSynchronize(stream_));
+  waitStream();
   return p;
 }
 

@@ -221,6 +221,7 @@ class Solver {
   void noteRuns();                  // drop the runs known to have completed
   bool settled();                   // after the stream is synchronised
   void settleRun();
+  void waitStream();
   void settle();
   // state fields (bits: Ux, Uy, Vx, Vy) a lost run left invalid and nobody has
   // set since
