@@ -2378,10 +2378,11 @@ int march2_segments(int nX, int nY, int rows, int rve, int4* out) {
 // r = n % 8, tile_of_block), and an XCD starts its workgroups in index
 // order.  Two measures shorten the end of a launch, where few workgroups
 // are left (20 x 1024^2, four stages on two waves):
-//  * column-edge segments first in each XCD's share: they run about a third
-//    longer than interior ones (123 against 90 us), and started first they
-//    leave workgroups of more even length for the end (3% shorter launches;
-//    moving the row-edge segments forward as well gains less);
+//  * column-edge segments first in each XCD's share: they run longer than
+//    interior ones (1.2 times; 123 against 90 us when this order was chosen,
+//    3% shorter launches then), and started first they leave workgroups of
+//    more even length for the end (moving the row-edge segments forward as
+//    well gains less);
 //  * the last twelfth of each share cut into shorter segments, so the last
 //    workgroups to start end sooner: halves, and quarters for the last
 //    forty-eighth (2.6% and 0.8% more; cutting a sixteenth or an eighth

@@ -3,8 +3,8 @@
 // The GPU's registers hold what the other kernels stream through HBM: each
 // workgroup of up to eight waves keeps U and V of one tile of an RVE in
 // registers for n iterations.  An iteration reads and writes no field and needs
-// no launch.  What bounds it: VALU issue of the tile (FP64, and split on grids
-// that fill the CUs), and the exchange between tiles -- a store reaches the
+// no launch.  What bounds it: the dependent chain of a wave's instructions at two
+// waves to a SIMD, and the exchange between tiles -- a store reaches the
 // memory both XCDs see in about 0.5 us and is read from there in about 1 us --
 // which is why a tile computes T = 2 iterations between exchanges, on a halo
 // of 2T nodes that it takes over from its neighbours.
@@ -12,9 +12,13 @@
 // us per iteration, single RVE (tile kernel, one iteration a launch, before there
 // were resident runs; chain kernels; here):
 //            64^2             256^2            333^2            512^2
-//   FP64     7.5 / 4.7 / 4.1  6.8 / 5.4 / 4.0  7.3 / 5.8 / 4.2  8.9 / 6.9 / 6.2
-//   split    6.8 / 3.1 / 2.6  6.0 / 3.3 / 2.6  6.5 / 3.9 / 3.0  7.2 / 4.3 / 3.9
-// T = 1 took 4.3 (FP64) and 3.1 (split) on the small grids.
+//   FP64     7.5 / 4.8 / 3.9  6.8 / 5.4 / 3.9  7.3 / 5.8 / 4.1  8.9 / 6.7 / 6.1
+//   split    6.8 / 3.1 / 2.6  6.0 / 3.3 / 2.6  6.5 / 3.9 / 3.1  7.2 / 4.1 / 3.9
+// One exchange an iteration (T = 1) on the same tiles: FP64 4.15, 4.5 and 4.6,
+// split 3.25, 3.6 and 3.8 at 64^2, 256^2 and 333^2.
+// The vector ALUs are busy 3% of the cycles at 64^2 (16 tiles), 33% at 333^2 in
+// split, 43% (FP64) and 36% (split) at 512^2 with a tile on nearly every CU; waves
+// wait half their life.
 //
 // Layout.  Lane L of every wave is column s+L of the tile's region, wave v
 // holds rows jr + v R .. jr + v R + R - 1 of it: the tile's own nodes and 2T
