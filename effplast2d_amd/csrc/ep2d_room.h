@@ -23,6 +23,23 @@ struct RoomUser {
                                      // or need not be (a batch in a step)
 };
 
+// While a stream is being captured, waiting for another stream, or asking it, is
+// refused and ends the capture; a thread in the relaxed mode may do both.  For
+// the library's own streams, of which none is being captured then.
+class RelaxedCapture {
+ public:
+  RelaxedCapture() { on_ = hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess; }
+  ~RelaxedCapture() {
+    if (on_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+  }
+  RelaxedCapture(const RelaxedCapture&) = delete;
+  RelaxedCapture& operator=(const RelaxedCapture&) = delete;
+
+ private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+  bool on_ = false;
+};
+
 // The words: the last run that has completed, and how a run failed (0: none did).
 inline bool run_ended(const unsigned* told, unsigned run) {
   return __atomic_load_n(told, __ATOMIC_ACQUIRE) == run ||
@@ -116,6 +133,7 @@ class DeviceRoom {
   static bool busy(RoomUser& u) {
     if (u.run != 0 && run_ended(u.told, u.run)) u.run = 0;
     if (u.atWork && !u.held) {
+      const RelaxedCapture relaxed;
       if (hipStreamQuery(u.stream) == hipSuccess) u.atWork = false;
       else (void)hipGetLastError();
     }

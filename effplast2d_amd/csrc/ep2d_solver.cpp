@@ -590,7 +590,11 @@ void Solver::settleRun() {
   if (!resRuns_.empty()) noteRuns();
   if (resRuns_.empty()) return;
   EP2D_HIP(hipSetDevice(device_));
-  waitStream();
+  {
+    // (iterate and applyAffine are queued beside a capture too)
+    const RelaxedCapture relaxed;
+    waitStream();
+  }
   settled();
 }
 

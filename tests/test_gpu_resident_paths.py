@@ -445,3 +445,34 @@ def test_a_batch_keeps_its_share(nX, resident):
     assert busy and runs == (resident, 0, 0)
     assert [r["status"] for r in state["out"]] == [0] * 8
     _same(a, _tiles(nX, "fp64", pa, init, 100))
+
+
+def test_handles_beside_a_capture():
+    """While a caller's stream is captured (in the mode that watches every thread),
+    handles on streams of their own go on, and ask which of them are at work."""
+    nX = 96
+    print("handles beside a capture", flush=True)
+    pa, init = _case(nX, "fp64", 8)
+    st = torch.cuda.Stream()
+    with EffPlast2D(pa, nX, nTasks=3, mode="fp64", stream=st.cuda_stream) as c, \
+            EffPlast2D(pa, nX, nTasks=3, mode="fp64") as a, \
+            EffPlast2D(pa, nX, nTasks=3, mode="split") as b, \
+            EffPlast2D(pa, nX, nTasks=3, mode="fp64", marchRows=16) as d:
+        for h in (a, c, d):
+            _start(h, init)
+        for h in (a, b, c, d):
+            h.iterate(32)       # (the first launches of the kernels load them)
+            h.sync()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=st, capture_error_mode="global"):
+            for n in (32, 5, 3, 200):   # the second waits for the first
+                for h in (d, a, b):
+                    h.iterate(n)
+            a.apply_affine(0.0, 0.0, 0.0, 0.0)
+            c.iterate(32)
+        for _ in range(2):
+            graph.replay()
+            torch.cuda.synchronize()
+        _same({k: c.get(k) for k in FIELDS}, _tiles(nX, "fp64", pa, init, 96))
+        for h in (a, d):
+            _same({k: h.get(k) for k in FIELDS}, _tiles(nX, "fp64", pa, init, 272))
