@@ -3,8 +3,10 @@
 #pragma once
 
 #include <algorithm>
+#include <chrono>
 #include <map>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 #include "ep2d_internal.h"
@@ -21,6 +23,8 @@ struct RoomUser {
   bool atWork = false;               // other work may be in flight
   bool held = false;                 // its stream must not be asked (a capture is on),
                                      // or need not be (a batch in a step)
+  std::thread::id thread;            // the thread it was last used by, and when;
+  std::chrono::steady_clock::time_point used, asked;  // when its stream was last asked
 };
 
 // While a stream is being captured, waiting for another stream, or asking it, is
@@ -81,12 +85,13 @@ class DeviceRoom {
   // 151 and 15).
   int enter(RoomUser* me, unsigned run, unsigned cus) {
     const std::lock_guard<std::mutex> lock(m_);
+    touch(me);
     int n = 1;
     bool all = run != 0, shared = false;
     std::vector<const RoomUser*> at;
     for (RoomUser* u : users_) {
       if (run == 0 && n >= 3) break;
-      if (u == me || !busy(*u)) continue;
+      if (u == me || !busy(*u, *me)) continue;
       n++;
       at.push_back(u);
       shared = shared || u->half + u->whole == 0;
@@ -110,12 +115,14 @@ class DeviceRoom {
   // Before launches that do not depend on the others'.
   void work(RoomUser* me) {
     const std::lock_guard<std::mutex> lock(m_);
+    touch(me);
     me->run = 0;
     me->atWork = true;
   }
   // The stream of `me` has been waited for.
   void idle(RoomUser* me) {
     const std::lock_guard<std::mutex> lock(m_);
+    touch(me);
     me->run = 0;
     me->atWork = false;
   }
@@ -130,14 +137,29 @@ class DeviceRoom {
   }
 
  private:
-  static bool busy(RoomUser& u) {
+  // Whether u is at work, seen from `me`, which has just been touched.  A stream
+  // takes about 5 us to answer, as long as a short call takes, so it is asked
+  // only so often.  A handle that another thread used a moment ago counts as at
+  // work between its calls too: 4 FP64 handles of 512^2 on a thread each, 40
+  // iterations and a residual a call, took 220 us a call while each went
+  // resident whenever the others were between calls (on tiles 151, on chains
+  // for several throughout 130).  Handles of one thread, waited for in turn, do
+  // not see each other.
+  static bool busy(RoomUser& u, const RoomUser& me) {
+    using std::chrono::microseconds;
     if (u.run != 0 && run_ended(u.told, u.run)) u.run = 0;
-    if (u.atWork && !u.held) {
+    if (u.atWork && !u.held && me.used - u.asked >= microseconds(300)) {
+      u.asked = me.used;
       const RelaxedCapture relaxed;
       if (hipStreamQuery(u.stream) == hipSuccess) u.atWork = false;
       else (void)hipGetLastError();
     }
-    return u.run != 0 || u.atWork;
+    return u.run != 0 || u.atWork ||
+           (u.thread != me.thread && me.used - u.used < microseconds(2000));
+  }
+  static void touch(RoomUser* me) {
+    me->thread = std::this_thread::get_id();
+    me->used = std::chrono::steady_clock::now();
   }
   std::mutex m_;
   std::vector<RoomUser*> users_;

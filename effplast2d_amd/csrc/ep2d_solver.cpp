@@ -354,7 +354,7 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
       // on the device (the kernel reads the current buffer as parity ^ cur)
       marchRows_ = opt_.marchRows;
       nSegs_ = march_segments(nX, nY, marchRows_, 0, nullptr);
-      std::vector<int4> segs((size_t)nSegs_), s2[kLoads], c3[kLoads], c2[kLoads];
+      std::vector<int4> segs((size_t)nSegs_), s2[kLoads], c3, c2;
       march_segments(nX, nY, marchRows_, 0, segs.data());
       const int2 dims = make_int2(nX, nY);
       const bool f32 = mode_ == EP2D_MODE_SPLIT;
@@ -369,7 +369,6 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
         // the 5 of this rule, 2.5 on the tile kernel; 512^2 7 on 4 rows, 3.1 on
         // the 16 of this rule, 4.1 on the tile kernel)
         const int rows = q == 0 ? marchRows_ : chain_rows(nX, nY, res / (q + 1));
-        segsFor_[q].rows = rows;
         auto segsOf = [&](int4* out) {
           if (ipl_ == 2) return march2_segments(nX, nY, rows, 0, out);
           if (wide_) return wide_segments(ipl_, nX, nY, rows, 0, out);
@@ -381,17 +380,17 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
                                       : raw));
         segsOf(s2[q].data());
         if (ordered) chain_work_order(s2[q].data(), raw, stageWaves_, &dims, res, s2[q].data());
-        if (ipl_ < 3) continue;
+        if (ipl_ < 3 || q > 0) continue;  // (one closing launch a call)
         // closing launches of 26 and 42 rows, of fewer on a small grid
         const int r2 = tileSingles_ ? std::min(26, rows) : 26;
         const int r3 = tileSingles_ ? std::min(42, rows) : 42;
-        c2[q].resize((size_t)march2_segments(nX, nY, r2, 0, nullptr));
-        march2_segments(nX, nY, r2, 0, c2[q].data());
+        c2.resize((size_t)march2_segments(nX, nY, r2, 0, nullptr));
+        march2_segments(nX, nY, r2, 0, c2.data());
         if (ipl_ == 4) {
           const int raw3 = chain_segments(3, nX, nY, r3, 0, nullptr, 1);
-          c3[q].resize((size_t)chain_work_order(nullptr, raw3, 1, &dims, res3, nullptr));
-          chain_segments(3, nX, nY, r3, 0, c3[q].data(), 1);
-          chain_work_order(c3[q].data(), raw3, 1, &dims, res3, c3[q].data());
+          c3.resize((size_t)chain_work_order(nullptr, raw3, 1, &dims, res3, nullptr));
+          chain_segments(3, nX, nY, r3, 0, c3.data(), 1);
+          chain_work_order(c3.data(), raw3, 1, &dims, res3, c3.data());
         }
       }
       std::vector<ResTile> tiles;
@@ -408,27 +407,19 @@ void Solver::init(const double pa[EP2D_NPARS], hipStream_t stream) {
       };
       auto putSegs = [&](const std::vector<int4>& v) { return put(v.data(), v.size() * sizeof(int4)); };
       const size_t atRve = put(&rd, sizeof(rd)), atSegs = putSegs(segs);
-      size_t at[kLoads][3];
-      for (int q = 0; q < kLoads; q++) {
-        at[q][0] = putSegs(s2[q]);
-        at[q][1] = putSegs(c3[q]);
-        at[q][2] = putSegs(c2[q]);
-      }
+      const size_t atC3 = putSegs(c3), atC2 = putSegs(c2);
+      size_t at[kLoads];
+      for (int q = 0; q < kLoads; q++) at[q] = putSegs(s2[q]);
       const size_t atTiles = put(tiles.data(), tiles.size() * sizeof(ResTile));
       // (after the tables: the record and exchange buffer of resident runs)
       const size_t resBytes = resTiles_ ? 256 + 2 * (size_t)resXpar_ : 0;
       char* blk = (char*)alloc(host.size() + resBytes);
       dRve_ = (RveDev*)(blk + atRve);
       dSegs_ = (int4*)(blk + atSegs);
-      for (int q = 0; q < kLoads; q++) {
-        Segments& g = segsFor_[q];
-        g.n = (int)s2[q].size();
-        g.n3 = (int)c3[q].size();
-        g.n2 = (int)c2[q].size();
-        g.d = (int4*)(blk + at[q][0]);
-        g.d3 = (int4*)(blk + at[q][1]);
-        g.d2 = (int4*)(blk + at[q][2]);
-      }
+      for (int q = 0; q < kLoads; q++)
+        segsFor_[q] = {(int)s2[q].size(), (int4*)(blk + at[q])};
+      close3_ = {(int)c3.size(), (int4*)(blk + atC3)};
+      close2_ = {(int)c2.size(), (int4*)(blk + atC2)};
       dResTiles_ = (ResTile*)(blk + atTiles);
       if (resTiles_) {
         dResCtl_ = (ResCtl*)(blk + host.size());
@@ -491,9 +482,12 @@ bool Solver::residentFits(long n) {
 // (0) on the other kernels, whose segments are those for the handles at work.
 int Solver::enterRoom(unsigned run, long n) {
   int at = 1;
-  if (inRoom_ && run == 0 && (n <= 1 || !tileSingles_)) inRoom_->work(&room_);
+  // (up to ipl_ iterations: closing launches and single ones only)
+  if (inRoom_ && run == 0 && (n <= ipl_ || !tileSingles_)) inRoom_->work(&room_);
   else if (inRoom_) at = inRoom_->enter(&room_, run, cus_);
-  load_ = tileSingles_ ? std::clamp(at, 1, kLoads) - 1 : 0;
+  // (a short call is mostly the latency of its launches: one handle's heights, or
+  // two handles', serve it better than many's)
+  load_ = tileSingles_ ? std::clamp(at, 1, n < kResMinIters ? 2 : kLoads) - 1 : 0;
   return at;
 }
 
@@ -949,11 +943,11 @@ void Solver::iterateLaunches(long n) {
   for (long q = 0; q < d; q++) launchMulti((int)(q & 1));
   // four closing iterations run as a three-iteration launch and the single,
   // three as a two-iteration launch and the single (the same results)
-  if (singles == 4 && segsFor_[load_].n3 > 0) {
+  if (singles == 4 && close3_.n > 0) {
     launchClose(3, (int)(d & 1));
     d++;
     singles = 1;
-  } else if (singles == 3 && segsFor_[load_].n2 > 0) {
+  } else if (singles == 3 && close2_.n > 0) {
     launchClose(2, (int)(d & 1));
     d++;
     singles = 1;
@@ -966,12 +960,11 @@ void Solver::iterateLaunches(long n) {
 // closing a run of multi-iteration launches; V is read from buffer
 // vIdx_ ^ q and written to the other, as in launchMulti.
 void Solver::launchClose(int ns, int q) {
-  const Segments& g = segsFor_[load_];
   if (ns == 3)
-    launch_chain(3, dRve_, g.d3, g.n3, iterMode(), cur_, vIdx_ ^ q, stream_, nullptr,
+    launch_chain(3, dRve_, close3_.d, close3_.n, iterMode(), cur_, vIdx_ ^ q, stream_, nullptr,
                  nullptr, 1);
   else
-    launch_march2(dRve_, g.d2, g.n2, iterMode(), cur_, vIdx_ ^ q, stream_, nullptr,
+    launch_march2(dRve_, close2_.d, close2_.n, iterMode(), cur_, vIdx_ ^ q, stream_, nullptr,
                   nullptr, true);
   cur_ ^= 1;
   stressStale_ = true;

@@ -178,17 +178,16 @@ class Solver {
   int ipl_ = 1;                     // iterations per launch: 1, 2 (pairs), 3 or 4 (chains)
   bool wide_ = false;               // chains on two columns per lane (split scheme)
   int stageWaves_ = 1;              // chains: waves side by side per stage
-  // Segments of the multi-iteration launches, and of the three- and
-  // two-iteration ones that close a run of a four- or three-iteration shape
-  // (chains of three waves, 42 rows; wave pairs, 26 rows).  Grids below 1024^2 on
-  // the automatic shape have them for one, two, and
-  // three handles and more at work.
+  // Segments of the multi-iteration launches (grids below 1024^2 on the automatic
+  // shape have them for one, two, and three handles and more at work), and of
+  // the three- and two-iteration ones that close a run of a four- or
+  // three-iteration shape (chains of three waves, 42 rows; wave pairs, 26 rows).
   struct Segments {
-    int rows = 0, n = 0, n3 = 0, n2 = 0;
-    int4 *d = nullptr, *d3 = nullptr, *d2 = nullptr;
+    int n = 0;
+    int4* d = nullptr;
   };
   static constexpr int kLoads = 3;
-  Segments segsFor_[kLoads];
+  Segments segsFor_[kLoads], close3_, close2_;
   int load_ = 0;                    // the ones in use
   bool tileSingles_ = false;        // single iterations on the tile kernel
   int vIdx_ = 0;                    // velocity buffer holding the current V

@@ -311,8 +311,8 @@ def test_runs_queue_up(mode):
 
 @pytest.mark.parametrize("mode,nX", [("fp64", 256), ("split", 400), ("fp64", 700)])
 def test_many_handles_at_once(mode, nX):
-    """With several handles at work the chains take taller segments (one height
-    for two handles, one for more), closing launches with them."""
+    """With several handles at work the chains take taller segments: one height
+    for two handles, one for more."""
     print(f"many handles {mode} nX={nX}", flush=True)
     cases = [_case(nX, mode, 60 + k) for k in range(6)]
     hs = [EffPlast2D(pa, nX, nTasks=3, mode=mode) for pa, _ in cases]
